@@ -313,18 +313,18 @@ bool plan_decode(const ffai_attn_desc* d, bool allow_split, size_t max_ws, const
   return true;
 }
 
-// `vector_ok`: the operands admit the decode kernel's vector accesses (it has no element-wise
-// path; misaligned decode shapes take fwd_kernel).
+// `dma_ok`: f32, or K and V admit the 16-bit decode kernel's DMA (other 16-bit decode shapes take
+// fwd_kernel).
 // `max_ws`: the workspace available. Every split serves speed only, so a plan whose partials
 // would exceed it runs its split items in fewer pieces, or whole, instead.
-Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool vector_ok,
+Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
                size_t max_ws = SIZE_MAX) {
   Plan p{};
   const Geometry geo = device_geometry();
   const int64_t cus = geo.cus;
   p.cus = geo.cus;
   p.xcd_shift = std::max(0, xcd_shift_of(geo.xcds));
-  if (vector_ok && plan_decode(d, allow_split, max_ws, geo, &p)) return p;
+  if (dma_ok && plan_decode(d, allow_split, max_ws, geo, &p)) return p;
   const int64_t bh = (int64_t)d->batch * d->heads_q;
   const bool f32 = d->q_dtype == FFAI_F32;
   const int n_tiles = (d->kv_len + ffai::kBlockN - 1) / ffai::kBlockN;
@@ -477,7 +477,8 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool vector_ok,
 
 // Workspace for a descriptor whatever the operands' alignment turns out to be.
 size_t plan_ws_bytes(const ffai_attn_desc* d) {
-  return std::max(make_plan(d, true, true).ws_bytes, make_plan(d, true, false).ws_bytes);
+  const size_t dma = make_plan(d, true, true).ws_bytes;
+  return d->q_dtype == FFAI_F32 ? dma : std::max(dma, make_plan(d, true, false).ws_bytes);
 }
 
 // ---- allocation-free entry point: a library-owned split-key scratch per device ----------------
@@ -534,15 +535,13 @@ int run_fwd(const ffai_attn_desc* d, const void* q, const void* k, const void* v
 
   const bool f32 = d->q_dtype == FFAI_F32;
   const bool kt = d->k_layout == FFAI_K_TRANSPOSED;
-  // The kernels' vector accesses: Q rows 16 B (4 f32 or 8 16-bit elements); K rows and V rows
-  // 16 B in the 16-bit kernels, 4 elements in the f32 kernel; K^T rows 4 keys; O 4 elements.
-  const int need_q = f32 ? 4 : 8, need_kv = f32 ? 4 : 8, need_k = kt ? 4 : need_kv;
-  const bool aligned = vec_of(q, qs, d->q_strides, need_q) == need_q &&
-                       vec_of(k, ks, d->k_strides, need_k) == need_k &&
-                       vec_of(v, ks, d->v_strides, need_kv) == need_kv &&
-                       vec_of(out, os, d->o_strides, 4) == 4;
+  // The 16-bit kernels' DMA of K and V tiles (global -> LDS): 16-byte rows, K^T rows 4 keys.
+  // Every other access is a vector access at element alignment.
+  const int need_k = kt ? 4 : 8;
+  const bool dma_ok = f32 || (vec_of(k, ks, d->k_strides, need_k) == need_k &&
+                              vec_of(v, ks, d->v_strides, 8) == 8);
 
-  const Plan pl = make_plan(d, allow_split, aligned, use_scratch ? kScratchBytes : SIZE_MAX);
+  const Plan pl = make_plan(d, allow_split, dma_ok, use_scratch ? kScratchBytes : SIZE_MAX);
   if (use_scratch && pl.ws_bytes > kScratchBytes)
     return fail(FFAI_ERR_WORKSPACE,
                 "this shape needs " + std::to_string(pl.ws_bytes) +
@@ -616,12 +615,11 @@ int run_fwd(const ffai_attn_desc* d, const void* q, const void* k, const void* v
   }
   p.xcd_remap = pl.xcd_remap ? 1 : 0;
   p.counters = static_cast<int32_t*>(ws);
-  p.aligned = aligned;
   {
     // the DMA path addresses a tile's rows by 32-bit byte offsets from the tile's first key
     const int64_t k_rows = kt ? d->head_dim : ffai::kBlockN;
     const int64_t lim = int64_t(1) << 31;
-    p.dma = aligned && !f32 && k_rows * d->k_strides[2] * 2 < lim &&
+    p.dma = dma_ok && !f32 && k_rows * d->k_strides[2] * 2 < lim &&
             int64_t(ffai::kBlockN) * d->v_strides[2] * 2 < lim;
   }
   p.scale_log2 = d->scale * 1.4426950408889634f;

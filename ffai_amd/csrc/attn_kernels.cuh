@@ -154,7 +154,6 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   const int tps = split < 0 ? n_tiles : (n_tiles + p.n_split - 1) / p.n_split;
   const int t_begin = split < 0 ? 0 : split * tps;
   const int t_end = min(n_tiles, t_begin + tps);
-  const bool aligned = p.aligned != 0;
 
   const QS* qp = reinterpret_cast<const QS*>(p.q) + b * p.q_sb + h * p.q_sh;
   const KVS* kp = reinterpret_cast<const KVS*>(p.k) + b * p.k_sb + hk * p.k_sh;
@@ -175,8 +174,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
       // step (j, e): lane group g supplies d = 8j + 4g + e
 #pragma unroll
       for (int j = 0; j < D / 8; ++j) {
-        const f32x4 x = aligned ? ld4f<kF32, true>(qr + 8 * j + 4 * g)
-                                : ld4f<kF32, false>(qr + 8 * j + 4 * g);
+        const f32x4 x = ld4f<kF32>(qr + 8 * j + 4 * g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) qf[c][4 * j + e] = ok ? x[e] : 0.f;
       }
@@ -184,7 +182,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
       // step s: lane group g supplies d = 16s + 8g .. +7
 #pragma unroll
       for (int s = 0; s < D / 16; ++s) {
-        const u32x4 x = aligned ? ld16(qr + 16 * s + 8 * g) : ld8h_elem(qr + 16 * s + 8 * g);
+        const u32x4 x = ld16h(qr + 16 * s + 8 * g);
         qf[c][s] = ok ? x : u32x4{0u, 0u, 0u, 0u};
       }
     }
@@ -194,8 +192,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   // f32:    K rows -> units of 4 elements; K^T -> 4 d-rows x 4 keys (transposed in registers);
   //         V -> 4 keys x 4 d (transposed in registers).
   // 16-bit: K rows, K^T rows and V rows -> units of 8 elements (one 128-bit LDS store each);
-  //         K^T rows are only 8-byte aligned in general (row stride = key count), so they are
-  //         read from global memory as two 8-byte halves.
+  //         K^T rows are only element-aligned in general (row stride = key count).
   constexpr int K_UNITS = F32 ? (KT ? (D / 4) * (BN / 4) : BN * (D / 4))
                               : (KT ? D * (BN / 8) : BN * (D / 8));
   constexpr int V_UNITS = F32 ? (BN / 4) * (D / 4) : BN * (D / 8);
@@ -223,15 +220,15 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   (void)swz_v;
   (void)swz_kr;
 
-  // Load tile `it` into kreg/vreg. Interior tiles of an aligned launch take unconditional
-  // vector loads (the uniform `full` branch); tail tiles clamp every index to the last valid key,
+  // Load tile `it` into kreg/vreg. Interior tiles take unconditional vector loads (the uniform
+  // `full` branch), at whatever alignment; tail tiles clamp every index to the last valid key,
   // so they too read only valid addresses without divergent branches. Rows past the last key are
   // zeroed by store_tile (K^T tails, loaded element-wise, are zeroed here): no value loaded here
   // is used before the tile is stored.
   auto load_tile = [&](int it) {
     const int kb = it * BN;
     const int klast = kv_end - 1;
-    const bool full = aligned && (kb + BN <= kv_end);
+    const bool full = kb + BN <= kv_end;
 #pragma unroll
     for (int i = 0; i < K_PER; ++i) {
       const int u = tid + i * NT;
@@ -244,7 +241,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
             const KVS* row = kp + (int64_t)(4 * d4 + r) * p.k_st;
             f32x4 x;
             if (full) {
-              x = ld4f<KVT, true>(row + key0);
+              x = ld4f<KVT>(row + key0);
             } else {
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
@@ -260,7 +257,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
         } else {
           const int key = kb + u / (D / 4), c = u % (D / 4);
           const KVS* src = kp + (int64_t)min(key, klast) * p.k_st + 4 * c;
-          kreg[i] = aligned ? ld4f<KVT, true>(src) : ld4f<KVT, false>(src);
+          kreg[i] = ld4f<KVT>(src);
         }
       } else {
         if constexpr (KT) {
@@ -269,8 +266,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
           const uint16_t* row = kp + (int64_t)d * p.k_st;
           u32x4 x;
           if (full) {
-            const u32x2 lo = ld8(row + key0), hi = ld8(row + key0 + 4);
-            x = u32x4{lo.x, lo.y, hi.x, hi.y};
+            x = ld16h(row + key0);
           } else {
             uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -284,7 +280,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
         } else {
           const int key = kb + u / (D / 8), c = u % (D / 8);
           const uint16_t* src = kp + (int64_t)min(key, klast) * p.k_st + 8 * c;
-          kreg[i] = aligned ? ld16(src) : ld8h_elem(src);
+          kreg[i] = ld16h(src);
         }
       }
     }
@@ -297,12 +293,12 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
         for (int r = 0; r < 4; ++r) {
           const int key = kb + 4 * k4 + r;
           const KVS* src = vp + (int64_t)min(key, klast) * p.v_st + 4 * d4;
-          vreg[4 * i + r] = aligned ? ld4f<KVT, true>(src) : ld4f<KVT, false>(src);
+          vreg[4 * i + r] = ld4f<KVT>(src);
         }
       } else {
         const int key = kb + u / (D / 8), c = u % (D / 8);
         const uint16_t* src = vp + (int64_t)min(key, klast) * p.v_st + 8 * c;
-        vreg[i] = aligned ? ld16(src) : ld8h_elem(src);
+        vreg[i] = ld16h(src);
       }
     }
   };
@@ -414,7 +410,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
     }
   };
   // Stage tile `it` into K buffer `kbuf` and V buffer `vbuf`: by DMA when whole and aligned,
-  // else through registers (clamped, zero-filled tail; element-wise loads when misaligned),
+  // else through registers (clamped, zero-filled tail; any alignment),
   // synchronously.
   auto stage_tile = [&](int kbuf, int vbuf, int it) {
     if (p.dma && it * BN + BN <= kv_end) {
@@ -1128,8 +1124,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
       for (int r = 0; r < 4; ++r) {
         const f32x4 x = {oacc[c][dt][4 * r] * inv, oacc[c][dt][4 * r + 1] * inv,
                          oacc[c][dt][4 * r + 2] * inv, oacc[c][dt][4 * r + 3] * inv};
-        if (aligned) st4<OUTT, true>(op + 32 * dt + 8 * r + 4 * g, x);
-        else st4<OUTT, false>(op + 32 * dt + 8 * r + 4 * g, x);
+        st4<OUTT>(op + 32 * dt + 8 * r + 4 * g, x);
       }
   }
 #ifdef FFAI_STAMPS

@@ -43,9 +43,9 @@ struct FwdParams {
   int32_t xcd_remap;
   int32_t xcd_shift;         // log2 of the device's XCD count (sections are whole XCD rounds)
   int32_t cus;               // the device's CUs (host side: launch shaping)
-  int32_t aligned;           // every operand admits the kernels' vector loads and stores
-  int32_t dma;               // 16-bit: whole tiles may go global -> LDS by DMA (aligned, and
-                             // each lane's byte offset within a K or V tile fits 32 bits)
+  int32_t dma;               // 16-bit: whole tiles may go global -> LDS by DMA (K and V aligned,
+                             // and each lane's byte offset within one of their tiles fits 32
+                             // bits)
   float scale_log2;          // scale * log2(e)
   int32_t o_pair;            // head_dim 64, 16-bit output whose rows admit 16-byte stores: a
                              // lane and its partner (lane ^ 32) exchange halves and store whole
@@ -56,8 +56,8 @@ struct FwdParams {
 #endif
 };
 
-// A decode launch: at most 32 query rows (group x Tq) per (batch, kv-head) unit, operands that
-// admit 16-byte Q/K/V row accesses (8-byte K^T rows) and 4-element output stores.
+// A decode launch: at most 32 query rows (group x Tq) per (batch, kv-head) unit; 16-bit: K and V
+// that admit the DMA's 16-byte row accesses (8-byte K^T rows).
 struct DecodeParams {
   const void* q;
   const void* k;

@@ -91,7 +91,6 @@ __global__ __launch_bounds__(256, 2) void fwd16_kernel(FwdParams p) {
   const int tps = split < 0 ? n_tiles : (n_tiles + p.n_split - 1) / p.n_split;
   const int t_begin = split < 0 ? 0 : split * tps;
   const int t_end = min(n_tiles, t_begin + tps);
-  const bool aligned = p.aligned != 0;
 
   const uint16_t* qp = reinterpret_cast<const uint16_t*>(p.q) + b * p.q_sb + h * p.q_sh;
   const uint16_t* kp = reinterpret_cast<const uint16_t*>(p.k) + b * p.k_sb + hk * p.k_sh;
@@ -108,7 +107,7 @@ __global__ __launch_bounds__(256, 2) void fwd16_kernel(FwdParams p) {
     const uint16_t* qr = qp + (int64_t)min(row, p.Tq - 1) * p.q_st;
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
-      const u32x4 x = aligned ? ld16(qr + 32 * s + 8 * g) : ld8h_elem(qr + 32 * s + 8 * g);
+      const u32x4 x = ld16h(qr + 32 * s + 8 * g);
       qf[c][s] = ok ? x : u32x4{0u, 0u, 0u, 0u};
     }
   }
@@ -131,7 +130,7 @@ __global__ __launch_bounds__(256, 2) void fwd16_kernel(FwdParams p) {
   auto load_tile = [&](int it) {
     const int kb = it * BN;
     const int klast = kv_end - 1;
-    const bool full = aligned && (kb + BN <= kv_end);
+    const bool full = kb + BN <= kv_end;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int u = tid + i * NT;
@@ -140,8 +139,7 @@ __global__ __launch_bounds__(256, 2) void fwd16_kernel(FwdParams p) {
         const int key0 = kb + 8 * kc;
         const uint16_t* row = kp + (int64_t)d * p.k_st;
         if (full) {
-          const u32x2 lo = ld8(row + key0), hi = ld8(row + key0 + 4);
-          kreg[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+          kreg[i] = ld16h(row + key0);
         } else {
           uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -154,11 +152,11 @@ __global__ __launch_bounds__(256, 2) void fwd16_kernel(FwdParams p) {
       } else {
         const int key = kb + u / (D / 8), c = u % (D / 8);
         const uint16_t* src = kp + (int64_t)min(key, klast) * p.k_st + 8 * c;
-        kreg[i] = aligned ? ld16(src) : ld8h_elem(src);
+        kreg[i] = ld16h(src);
       }
       const int key = kb + u / (D / 8), c = u % (D / 8);
       const uint16_t* src = vp + (int64_t)min(key, klast) * p.v_st + 8 * c;
-      vreg[i] = aligned ? ld16(src) : ld8h_elem(src);
+      vreg[i] = ld16h(src);
     }
   };
   auto store_tile = [&](int buf, int it) {
@@ -630,8 +628,7 @@ __global__ __launch_bounds__(256, 2) void fwd16_kernel(FwdParams p) {
 #pragma unroll
     for (int db = 0; db < 4; ++db) {
       const f32x4 x = oacc[c][db] * inv;
-      if (aligned) st4<OUTT, true>(op + 16 * db + 4 * g, x);
-      else st4<OUTT, false>(op + 16 * db + 4 * g, x);
+      st4<OUTT>(op + 16 * db + 4 * g, x);
     }
   }
 }

@@ -33,7 +33,7 @@ __device__ __forceinline__ void store_row_chunk(const DecodeParams& p, int b, in
   const int h = hk * p.group + n / p.Tq, t = n % p.Tq;
   store_t<OUTT>* op = reinterpret_cast<store_t<OUTT>*>(p.o) + b * p.o_sb + h * p.o_sh +
                       (int64_t)t * p.o_st + 4 * c4;
-  st4<OUTT, true>(op, acc * inv);
+  st4<OUTT>(op, acc * inv);
 }
 
 // The end of a decode unit's workgroup, shared by the decode kernels: merge the NWD waves'
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
         const int k4 = kb + 8 * kc;
         const uint16_t* row = kp + (int64_t)d * p.k_st;
         const bool v0 = k4 + 3 <= klast, v1 = k4 + 7 <= klast;
-        const u32x2 lo = ld8(row + (v0 ? k4 : 0)), hi = ld8(row + (v1 ? k4 + 4 : 0));
+        const u32x2 lo = ld8h(row + (v0 ? k4 : 0)), hi = ld8h(row + (v1 ? k4 + 4 : 0));
         kreg[j] = u32x4{v0 ? lo.x : 0u, v0 ? lo.y : 0u, v1 ? hi.x : 0u, v1 ? hi.y : 0u};
       } else {
         const int key = kb + u / (D / 8), c = u % (D / 8);
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
     const uint16_t* qr = reinterpret_cast<const uint16_t*>(p.q) + b * p.q_sb +
                          h_row[c] * p.q_sh + (int64_t)t_row[c] * p.q_st;
 #pragma unroll
-    for (int h = 0; h < D / 32; ++h) qf[c][h] = ld16(qr + 32 * h + 8 * q4);
+    for (int h = 0; h < D / 32; ++h) qf[c][h] = ld16h(qr + 32 * h + 8 * q4);
   }
 
 #pragma unroll 1
@@ -635,7 +635,10 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
 //     groups' partial outputs are summed at the end.
 // Waves take their own 64-key tiles and merge through LDS; split units merge as in
 // decode_kernel (finish_unit). The host launches it for f32 queries, group x q_len == 1,
-// head_dim 64, 4-element-aligned operands, and heads whose K and V lie within 2^31 bytes.
+// head_dim 64, and heads whose K and V lie within 2^31 bytes. Operands need no more than element
+// alignment: a sequence's K^T rows are as long as its key count, so three steps in four leave
+// them off 16-byte boundaries (6 heads over 37 keys on the fused kernel, where such steps went
+// before: 12.9 us on the device; here 4.1)
 template <int KVT, bool KT, int NWD>
 __global__ __launch_bounds__(NWD * 64) void decode_vec_kernel(DecodeParams p) {
   constexpr int D = 64;
@@ -647,7 +650,8 @@ __global__ __launch_bounds__(NWD * 64) void decode_vec_kernel(DecodeParams p) {
   constexpr int VC = D / VE;         // chunks per V row: lanes per row group
   constexpr int VG = 64 / VC;        // row groups: 4 (f32) or 8 (16-bit)
   constexpr int VR = BN / VG;        // rows per group: 16 or 8
-  using KR = std::conditional_t<KVT == kF32, f32x4, u32x2>;  // 4 K elements as loaded
+  using KR = std::conditional_t<KVT == kF32, f32x4, u32x2>;      // 4 K elements as loaded
+  using KE = std::conditional_t<KVT == kF32, f32x4_e, u32x2_h>;  // (element-aligned)
   __shared__ __attribute__((aligned(16))) float mlds[NWD * WST];
   __shared__ __attribute__((aligned(16))) float wlds[NWD * BN];  // each wave's tile weights
 
@@ -679,7 +683,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_vec_kernel(DecodeParams p) {
   float q[16];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    const f32x4 x = *reinterpret_cast<const f32x4*>(qr + 4 * c);
+    const f32x4 x = ld4f<kF32>(qr + 4 * c);
 #pragma unroll
     for (int e = 0; e < 4; ++e) q[4 * c + e] = x[e];
   }
@@ -713,7 +717,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_vec_kernel(DecodeParams p) {
       if (kc0 + 4 <= p.Tk) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          kraw[i] = *reinterpret_cast<const KR*>(kb8 + off);
+          kraw[i] = *reinterpret_cast<const KE*>(kb8 + off);
           off += kstep;
           asm volatile("" : "+v"(off));
         }
@@ -740,7 +744,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_vec_kernel(DecodeParams p) {
       for (int r = 0; r < 4; ++r) {
         const KVS* kr = kp + (int64_t)min(k0 + r, kv_end - 1) * p.k_st + 16 * dg;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) kraw[4 * r + c] = *reinterpret_cast<const KR*>(kr + 4 * c);
+        for (int c = 0; c < 4; ++c) kraw[4 * r + c] = *reinterpret_cast<const KE*>(kr + 4 * c);
       }
     }
     u32x4 vx[VR];  // row VR vg + i, elements VE vc .. VE vc + VE - 1 (raw bits)
@@ -750,7 +754,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_vec_kernel(DecodeParams p) {
       if (kb + BN <= kv_end) {
 #pragma unroll
         for (int i = 0; i < VR; ++i) {
-          vx[i] = ld16(vb8 + off);
+          vx[i] = ld16h(vb8 + off);
           off += vstep;
           asm volatile("" : "+v"(off));
         }
@@ -759,7 +763,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_vec_kernel(DecodeParams p) {
 #pragma unroll
         for (int i = 0; i < VR; ++i) {
           const uint32_t row = (uint32_t)min(r0 + i, kv_end - 1);
-          vx[i] = ld16(vb8 + (row * (uint32_t)p.v_st + (uint32_t)(VE * vc)) * ES);
+          vx[i] = ld16h(vb8 + (row * (uint32_t)p.v_st + (uint32_t)(VE * vc)) * ES);
         }
       }
     }

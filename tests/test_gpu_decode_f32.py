@@ -181,3 +181,34 @@ def test_graph_replay_matches_eager(gpu):
         torch.cuda.synchronize()
         assert torch.equal(out, eager), i
         fa.attention(q, kt, v, k_transposed=True, out=eager)  # eager work between replays
+
+
+@pytest.mark.parametrize("kv_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("k_transposed", [True, False])
+@pytest.mark.parametrize("keys", [37, 130, 1037])
+def test_element_aligned_operands(gpu, kv_dtype, k_transposed, keys):
+    """Q, K, V and O one element off 16-byte boundaries, K^T rows of an odd length: the same
+    vector accesses at element alignment, still on the decode kernel."""
+    rng = np.random.default_rng(350 + keys)
+    h = 6
+    q = randn(rng, (1, h, 1, 64))
+    k = randn(rng, (1, h, keys, 64))
+    v = randn(rng, (1, h, keys, 64))
+    if kv_dtype == torch.float16:
+        k, v = k.astype(np.float16).astype(np.float32), v.astype(np.float16).astype(np.float32)
+    want = oracle.attend_general(q, k, v, k_transposed=False, scale=0.125)
+
+    def shifted(x, dtype):
+        flat = torch.zeros(x.size + 1, dtype=dtype, device=gpu)
+        flat[1:] = _dev(x.reshape(-1), dtype, gpu)
+        return flat[1:].view(*x.shape)
+
+    qd = shifted(q, torch.float32)
+    kd = shifted(np.ascontiguousarray(np.swapaxes(k, 2, 3)) if k_transposed else k, kv_dtype)
+    vd = shifted(v, kv_dtype)
+    out = torch.zeros(h * 64 + 1, device=gpu)[1:].view(1, h, 1, 64)
+    assert _kernel_of(qd, kd, vd, out, k_transposed=k_transposed) == "decode"
+    fa.attention(qd, kd, vd, k_transposed=k_transposed, scale=0.125, out=out)
+    err = max_abs(out.cpu().numpy(), want)
+    print(f"element-aligned f32-query decode {kv_dtype} kt={k_transposed} {keys}: {err:.3e}")
+    assert err < TOL_F32
