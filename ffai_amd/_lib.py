@@ -108,6 +108,7 @@ def load():
     L.ffai_attn_workspace_bytes.argtypes = [dp, ctypes.POINTER(sz)]
     L.ffai_attn_fwd.argtypes = [dp, vp, vp, vp, vp, vp, sz, vp]
     L.ffai_attn_plan_info.argtypes = [dp, ctypes.POINTER(ctypes.c_int32)]
+    L.ffai_attn_row_block.argtypes = [dp]
     L.ffai_attn_fwd_noalloc.argtypes = [dp, vp, vp, vp, vp, vp]
     L.ffai_attn_noalloc_plan_info.argtypes = [dp, ctypes.POINTER(ctypes.c_int32),
                                               ctypes.POINTER(sz)]
@@ -157,7 +158,7 @@ def load():
     L.ffai_probe_pipes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp]
     for name in ("ffai_probe_empty", "ffai_probe_read", "ffai_probe_pipes", "ffai_attn_serves",
                  "ffai_attn_workspace_bytes", "ffai_attn_fwd",
-                 "ffai_attn_plan_info", "ffai_attn_plan_splits", "ffai_attn_fwd_noalloc",
+                 "ffai_attn_plan_info", "ffai_attn_row_block", "ffai_attn_plan_splits", "ffai_attn_fwd_noalloc",
                  "ffai_attn_noalloc_plan_info",
                  "ffai_serves",
                  "ffai_attend", "ffai_attend_workspace_bytes", "ffai_attend_merged",

@@ -156,6 +156,15 @@ int attn_variant() {
   return v;
 }
 
+// FFAI_ATTN_SPLITS (> 0) forces the pieces of every fwd item: a tuning knob.
+int forced_splits() {
+  static const int n = [] {
+    const char* e = std::getenv("FFAI_ATTN_SPLITS");
+    return e ? std::atoi(e) : 0;
+  }();
+  return n;
+}
+
 constexpr int kMinSeq = 256;  // flash_attn.rs:55 (MIN_SEQ)
 constexpr int kHD = 64;       // flash_attn.rs:50
 
@@ -233,6 +242,13 @@ struct Plan {
   size_t ws_bytes;
 };
 
+// 64-key tiles any row of the call may see.
+int key_tiles(const ffai_attn_desc* d) {
+  int64_t kv = d->kv_len;
+  if (d->causal) kv = std::min<int64_t>(kv, (int64_t)d->q_offset + d->q_len);
+  return (int)std::max<int64_t>(1, (kv + ffai::kBlockN - 1) / ffai::kBlockN);
+}
+
 // Decode launch: 16-bit inputs and at most 32 query rows per (batch, kv-head), so one MFMA
 // column block holds every row that reads a K/V head. Each wave of a workgroup takes one 64-key
 // tile. A unit with more tiles than its workgroup's waves is split over workgroups, whose
@@ -242,7 +258,7 @@ struct Plan {
 // `max_ws`: the workspace available; a split that would need more is coarsened (more tiles per
 // workgroup) until it fits, down to no split.
 // f32 queries take the f32 decode kernel (decode_vec_kernel: the reference's decode arms, one
-// query row per unit, head_dim 64); 16-bit ones the MFMA decode kernel (up to 32 rows).
+// query row per unit, head_dim 64); 16-bit ones the MFMA decode kernel.
 bool plan_decode(const ffai_attn_desc* d, bool allow_split, size_t max_ws, const Geometry& geo,
                  Plan* p) {
   const int group = d->heads_q / d->heads_kv;
@@ -265,9 +281,7 @@ bool plan_decode(const ffai_attn_desc* d, bool allow_split, size_t max_ws, const
       ((int64_t)d->head_dim * d->k_strides[2] + d->kv_len) * es >= lim)
     return false;
   const int64_t units = (int64_t)d->batch * d->heads_kv;
-  int64_t kv_blk = d->kv_len;
-  if (d->causal) kv_blk = std::min<int64_t>(kv_blk, (int64_t)d->q_offset + d->q_len);
-  const int64_t n_tiles = std::max<int64_t>(1, (kv_blk + ffai::kBlockN - 1) / ffai::kBlockN);
+  const int64_t n_tiles = key_tiles(d);
   // 16-bit kernel: LDS, 16 KB (32 KB at head_dim 128) a wave; f32 kernel: registers
   const int max_waves = (vec || d->head_dim == 64) ? 8 : 4;
   // A grid of at least kMinWorkgroups stays at max_waves tiles per workgroup; a smaller one is
@@ -311,6 +325,44 @@ bool plan_decode(const ffai_attn_desc* d, bool allow_split, size_t max_ws, const
   p->n_work = (int)(units * p->n_split);
   p->ws_bytes = split_bytes(tps);
   return true;
+}
+
+// Row blocks: 16-bit calls of more rows per (batch, kv-head) than a decode unit holds, on the decode
+// kernel in blocks of 16 or 32 rows, each over all its keys in one workgroup (the waves split the
+// keys and merge in LDS: no partials, no workspace). Returns the rows per block, or 0 where the
+// call runs its plan (make_plan) instead. `dma_ok` as there.
+// Taken by grids that fit one workgroup per CU: there fwd_kernel has too few waves, or must split
+// the keys over workgroups and merge through memory. 16-row blocks while they fit, else 32. us per
+// call, fwd_kernel / 16 / 32 rows (head_dim 64 unless said): 16 heads x 227 rows x 1500 keys
+// 15.0 / 8.8 / 11.3; x 300 rows (304 blocks of 16: a second round) 16.7 / 15.0 / 11.4; the same
+// causal over 448 keys 10.7 / 7.8 / 6.4; 12 heads x 600 x 600 12.8 / 11.6 / 8.9; 20 heads x 600 x
+// 600 (380 blocks of 32) 14.3 / 16.3 / 14.9.
+// A workgroup's time grows with its keys, which fwd_kernel spreads over the chip: up to 4096 keys
+// at head_dim 64 (8 waves; 6 heads x 40 rows 38.8 / 14.9 / 19.5; at 8192 keys and 16 heads x 64
+// rows 25.0 / 30.3 / 36.5); at head_dim 128 (4 waves) up to 3072 in 16-row blocks (16 heads x 64
+// rows 33.0 / 28.8 / 37.2, at 4096 34.9 / 43.0 / 55.2) and 1536 in 32-row ones (16 heads x 227
+// rows 27.9 / 17.1 / 20.9; 1 head x 2048 causal 26.4 / 22.2 / 28.3).
+// A forced launch shape or split (the tuning knobs) keeps the call on its plan.
+int row_block_of(const ffai_attn_desc* d, bool dma_ok) {
+  const int group = d->heads_q / d->heads_kv;
+  const int64_t rows = (int64_t)group * d->q_len;
+  if (d->q_dtype == FFAI_F32 || !dma_ok || rows <= 32) return 0;
+  if (d->k_layout == FFAI_K_TRANSPOSED && d->kv_len < 4) return 0;  // 4-key chunks
+  const int64_t lim = int64_t(1) << 31;  // as in plan_decode
+  if (int64_t(std::max(d->head_dim, ffai::kBlockN)) * d->k_strides[2] * 2 >= lim ||
+      int64_t(ffai::kBlockN) * d->v_strides[2] * 2 >= lim)
+    return 0;
+  if (g_split_items.load(std::memory_order_relaxed) != 0 || forced_splits() > 0 ||
+      attn_variant() >= 0 || decode_tiles_per_wg() > 0)
+    return 0;
+  const Geometry geo = device_geometry();
+  const int64_t units = (int64_t)d->batch * d->heads_kv;
+  const int64_t b16 = units * ((rows + 15) / 16), b32 = units * ((rows + 31) / 32);
+  const bool d64 = d->head_dim == 64;
+  const int n_tiles = key_tiles(d);
+  if (b16 <= geo.cus && n_tiles <= (d64 ? 64 : 48)) return 16;
+  if (b32 <= geo.cus && n_tiles <= (d64 ? 64 : 24)) return 32;
+  return 0;
 }
 
 // `dma_ok`: f32, or K and V admit the 16-bit decode kernel's DMA (other 16-bit decode shapes take
@@ -384,12 +436,7 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
   } else if (f32 && items < 4 * cus) {
     want = (16 * cus + 4 * items - 1) / (4 * items);
   }
-  // FFAI_ATTN_SPLITS (> 0) forces the pieces of every item: a tuning knob.
-  static const int forced_splits = [] {
-    const char* e = std::getenv("FFAI_ATTN_SPLITS");
-    return e ? std::atoi(e) : 0;
-  }();
-  if (forced_splits > 0) want = forced_splits;
+  if (forced_splits() > 0) want = forced_splits();
   int64_t lo = 0, hi = want > 1 ? items : 0;
   if (want == 1 && !f32) {
     // Long grids split only the items that would leave the GPU partly idle at the end.
@@ -541,7 +588,17 @@ int run_fwd(const ffai_attn_desc* d, const void* q, const void* k, const void* v
   const bool dma_ok = f32 || (vec_of(k, ks, d->k_strides, need_k) == need_k &&
                               vec_of(v, ks, d->v_strides, 8) == 8);
 
-  const Plan pl = make_plan(d, allow_split, dma_ok, use_scratch ? kScratchBytes : SIZE_MAX);
+  Plan pl;
+  const int row_block = row_block_of(d, dma_ok);
+  if (row_block) {
+    pl = Plan{};
+    pl.decode = true;
+    pl.tiles_per_split = key_tiles(d);
+    pl.waves = d->head_dim == 64 && pl.tiles_per_split > 4 ? 8 : 4;
+    pl.n_split = 1;
+  } else {
+    pl = make_plan(d, allow_split, dma_ok, use_scratch ? kScratchBytes : SIZE_MAX);
+  }
   if (use_scratch && pl.ws_bytes > kScratchBytes)
     return fail(FFAI_ERR_WORKSPACE,
                 "this shape needs " + std::to_string(pl.ws_bytes) +
@@ -582,6 +639,7 @@ int run_fwd(const ffai_attn_desc* d, const void* q, const void* k, const void* v
     p.Tq = d->q_len; p.Tk = d->kv_len;
     p.causal = d->causal; p.q_offset = d->q_offset;
     p.n_split = pl.n_split; p.tiles_per_split = pl.tiles_per_split; p.n_work = pl.n_work;
+    p.row_block = row_block;
     p.scale_log2 = d->scale * 1.4426950408889634f;
 #ifdef FFAI_STAMPS
     p.stamps = g_stamp_buf.load();
@@ -786,6 +844,14 @@ int ffai_attn_plan_info(const ffai_attn_desc* d, int32_t info[5]) {
   info[3] = p.tiles_per_split;
   info[4] = p.n_work;
   return FFAI_OK;
+}
+
+int ffai_attn_row_block(const ffai_attn_desc* d) {
+  std::string why;
+  const int rc = check_desc(d, &why);
+  if (rc == FFAI_DECLINED) return 0;
+  if (rc != FFAI_OK) return fail(rc, why);
+  return row_block_of(d, true);
 }
 
 int ffai_attn_noalloc_plan_info(const ffai_attn_desc* d, int32_t info[5], size_t* bytes) {

@@ -56,7 +56,7 @@ struct FwdParams {
 #endif
 };
 
-// A decode launch: at most 32 query rows (group x Tq) per (batch, kv-head) unit; 16-bit: K and V
+// A decode launch: at most 32 query rows (group x Tq) per (batch, kv-head) unit or row block; 16-bit: K and V
 // that admit the DMA's 16-byte row accesses (8-byte K^T rows).
 struct DecodeParams {
   const void* q;
@@ -70,11 +70,13 @@ struct DecodeParams {
   int64_t k_sb, k_sh, k_st;
   int64_t v_sb, v_sh, v_st;
   int64_t o_sb, o_sh, o_st;
-  int32_t B, Hkv, group, Tq, Tk;  // group = Hq / Hkv; rows per unit R = group * Tq <= 32
+  int32_t B, Hkv, group, Tq, Tk;  // group = Hq / Hkv; rows per unit group * Tq
   int32_t causal, q_offset;
   int32_t n_split;          // workgroups per unit
   int32_t tiles_per_split;  // 64-key tiles per workgroup
   int32_t n_work;           // B * Hkv * n_split
+  int32_t row_block;        // 0, or the rows (16 or 32) of a unit's row blocks: any number of
+                            // query rows, n_split 1
   float scale_log2;
 #ifdef FFAI_STAMPS
   uint64_t* stamps;         // diagnostic builds only: per-workgroup event times

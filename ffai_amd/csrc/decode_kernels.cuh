@@ -25,12 +25,20 @@
 namespace ffai {
 namespace {
 
-// Output row n (of the unit's R rows), chunk c4 of 4 elements, normalised by l.
-template <int OUTT, int D>
+// Output row n (of the unit's R rows), chunk c4 of 4 elements, normalised by l. RB: the unit is a
+// block of rows of its (batch, kv-head), the first one row0, positions outermost.
+template <int OUTT, int D, bool RB = false>
 __device__ __forceinline__ void store_row_chunk(const DecodeParams& p, int b, int hk, int n, int c4,
-                                                f32x4 acc, float l) {
+                                                f32x4 acc, float l, int row0 = 0) {
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  const int h = hk * p.group + n / p.Tq, t = n % p.Tq;
+  int h, t;
+  if constexpr (RB) {
+    t = p.group == 1 ? row0 + n : (row0 + n) / p.group;
+    h = hk * p.group + (row0 + n - t * p.group);
+  } else {
+    h = hk * p.group + n / p.Tq;
+    t = n % p.Tq;
+  }
   store_t<OUTT>* op = reinterpret_cast<store_t<OUTT>*>(p.o) + b * p.o_sb + h * p.o_sh +
                       (int64_t)t * p.o_st + 4 * c4;
   st4<OUTT>(op, acc * inv);
@@ -44,9 +52,10 @@ __device__ __forceinline__ void store_row_chunk(const DecodeParams& p, int b, in
 // MR * OROW + MR + n. Every thread of the workgroup calls it, after a barrier that publishes the
 // partials.
 // Returns true when this workgroup wrote the unit's rows (unsplit, or the unit's last split).
-template <int OUTT, int D, int NWD, int OROW, int MR, int WST>
+template <int OUTT, int D, int NWD, int OROW, int MR, int WST, bool RB = false>
 __device__ __forceinline__ bool finish_unit(const DecodeParams& p, const float* mbase, int b,
-                                            int hk, int unit, int split, int R, int tid) {
+                                            int hk, int unit, int split, int R, int tid,
+                                            int row0 = 0) {
   constexpr int C4 = D / 4;  // 4-float chunks per row
   const int items = R * C4;
   const int64_t prow0 = ((int64_t)unit * p.n_split + split) * R;  // this split's first partial row
@@ -77,8 +86,8 @@ __device__ __forceinline__ bool finish_unit(const DecodeParams& p, const float* 
       acc += wt * *reinterpret_cast<const f32x4*>(&mb[n * OROW + 4 * c4]);
       L = __builtin_fmaf(wt, mb[MR * OROW + MR + n], L);
     }
-    if (p.n_split == 1) {
-      store_row_chunk<OUTT, D>(p, b, hk, n, c4, acc, L);
+    if (RB || p.n_split == 1) {
+      store_row_chunk<OUTT, D, RB>(p, b, hk, n, c4, acc, L, row0);
     } else {
       // This split's partial, written with device-scope (sc1) buffer stores: each one reaches
       // the device's coherence point before it is acknowledged, so the unit's last workgroup
@@ -92,7 +101,7 @@ __device__ __forceinline__ bool finish_unit(const DecodeParams& p, const float* 
                                               kDeviceScope);
     }
   }
-  if (p.n_split == 1) return true;
+  if (RB || p.n_split == 1) return true;
 
   // ---- count this split; the unit's last one merges them all.
   // Ordering: every thread waits for its partial stores to be acknowledged (vmcnt(0): device-
@@ -157,7 +166,15 @@ __device__ __forceinline__ bool finish_unit(const DecodeParams& p, const float* 
 }
 
 // NC: 16-column blocks of query rows (1 for units of at most 16 rows, 2 for up to 32).
-template <int MODE, int OUTT, int D, bool KT, int NWD, int NC>
+// RB: more rows than that read the kv-head (a prompt), and a workgroup takes one block of 16 NC of
+// them, positions outermost, over all its keys (grid: kv-heads, row blocks, batch). The waves
+// still split the keys among themselves and merge in LDS, so that a short grid's long key range
+// costs no partials in memory. The row blocks of a head reread its K and V, so those loads keep
+// the default cache policy; with kv-heads innermost in the grid, a head's blocks fall on few XCDs
+// and share their L2. Bound by each wave's chain of load, products and softmax per tile (~1.9 us).
+// A prompt's cross-attention, 16 heads x 227 rows x 1500 keys: 15.0 us on fwd_kernel in 6 pieces,
+// 8.8 here; its causal self-attention 9.1 and 4.6.
+template <int MODE, int OUTT, int D, bool KT, int NWD, int NC, bool RB = false>
 __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   static_assert(MODE == kBF16 || MODE == kF16, "decode kernel reads 16-bit Q, K and V");
   // Per-wave LDS: one K tile ([key][d] or [d][key]) and one V tile ([key][d]), 16-bit, rows
@@ -180,8 +197,8 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   //      indices are the workgroup's own and its operand addresses are scalar arithmetic (a
   //      division of a flat index cost ~0.3 us of dependent vector instructions before the first
   //      K/V load could be issued)
-  const int split = wg_id_x();
-  const int hk = wg_id_y();
+  const int split = RB ? 0 : wg_id_x();
+  const int hk = RB ? wg_id_x() : wg_id_y();
   const int b = wg_id_z();
   const int unit = b * p.Hkv + hk;
 
@@ -193,26 +210,35 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q4 = lane >> 4;   // lane group: contraction elements 8 q4 .., accumulator rows 4 q4 ..
   const int n16 = lane & 15;  // this lane's column in each 16-column block
-  const int R = p.group * p.Tq;
+  const int row0 = RB ? wg_id_y() * 16 * NC : 0;
+  const int R = RB ? min(16 * NC, p.group * p.Tq - row0) : p.group * p.Tq;
   // the unit's query row of column c (block c / 16): n = 16 c + n16; columns past R repeat row
   // R - 1 (each column's scores, weights and sums stay in that column, and only the first R
   // are read back)
   int t_row[NC], h_row[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int rn = min(16 * c + n16, R - 1);
-    t_row[c] = rn % p.Tq;
-    h_row[c] = hk * p.group + rn / p.Tq;
+    const int rn = row0 + min(16 * c + n16, R - 1);
+    if constexpr (RB) {
+      t_row[c] = p.group == 1 ? rn : rn / p.group;
+      h_row[c] = hk * p.group + (rn - t_row[c] * p.group);
+    } else {
+      t_row[c] = rn % p.Tq;
+      h_row[c] = hk * p.group + rn / p.Tq;
+    }
   }
 
   int kv_end = p.Tk;
   if (p.kv_lens) kv_end = min(kv_end, max(0, p.kv_lens[b]));
   kv_end = __builtin_amdgcn_readfirstlane(kv_end);  // uniform (one batch item per workgroup)
   int kv_blk = kv_end;  // keys any row of the unit may see
-  if (p.causal) kv_blk = min(kv_end, max(0, p.q_offset + p.Tq));
+  if (p.causal) {
+    const int t_max = RB ? (p.group == 1 ? row0 + R - 1 : (row0 + R - 1) / p.group) : p.Tq - 1;
+    kv_blk = min(kv_end, max(0, p.q_offset + t_max + 1));
+  }
   const int n_tiles = (kv_blk + BN - 1) / BN;
-  const int t_begin = split * p.tiles_per_split;
-  const int t_end = min(n_tiles, t_begin + p.tiles_per_split);
+  const int t_begin = RB ? 0 : split * p.tiles_per_split;
+  const int t_end = RB ? n_tiles : min(n_tiles, t_begin + p.tiles_per_split);
   const int iters = t_end > t_begin ? (t_end - t_begin + NWD - 1) / NWD : 0;
   const float sl2 = p.scale_log2;
   int lim[NC];  // the last key column block c's row may see
@@ -275,13 +301,13 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
       const int r = j * KRB + kr;
       const uint32_t off =
           (uint32_t)(2 * (r * p.k_st + 8 * (KT ? swz_kt(r, kpc) : swz_kr(r, kpc))));
-      if (KT || j * KRB < valid) lds_dma16_sbase<true>(kbase, off, kla + j * 1024);
+      if (KT || j * KRB < valid) lds_dma16_sbase<!RB>(kbase, off, kla + j * 1024);
     }
 #pragma unroll
     for (int j = 0; j < VBUF / 512; ++j) {
       const int r = j * VRB + vr;
       const uint32_t off = (uint32_t)(2 * (r * p.v_st + 8 * swz_v(r, vpc)));
-      if (j * VRB < valid) lds_dma16_sbase<true>(vbase, off, vla + j * 1024);
+      if (j * VRB < valid) lds_dma16_sbase<!RB>(vbase, off, vla + j * 1024);
     }
   };
   // The operand's last tile, when it has at least 8 keys but fewer than 64 (cross-attention over
@@ -302,11 +328,11 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
         const int c0 = kb + 8 * swz_kt(r, kpc);
         const int src = c0 + 8 <= p.Tk ? c0 : kb;
         const uint32_t off = (uint32_t)(2 * (r * p.k_st + (src - kb)));
-        lds_dma16_sbase<true>(kbase, off, kla + j * 1024);
+        lds_dma16_sbase<!RB>(kbase, off, kla + j * 1024);
       } else {
         const int key = min(kb + r, klast);
         const uint32_t off = (uint32_t)(2 * ((key - kb) * p.k_st + 8 * swz_kr(r, kpc)));
-        lds_dma16_sbase<true>(kbase, off, kla + j * 1024);
+        lds_dma16_sbase<!RB>(kbase, off, kla + j * 1024);
       }
     }
 #pragma unroll
@@ -314,7 +340,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
       const int r = j * VRB + vr;
       const int key = min(kb + r, klast);
       const uint32_t off = (uint32_t)(2 * ((key - kb) * p.v_st + 8 * swz_v(r, vpc)));
-      lds_dma16_sbase<true>(vbase, off, vla + j * 1024);
+      lds_dma16_sbase<!RB>(vbase, off, vla + j * 1024);
     }
   };
   // The valid keys of the 8-key K^T chunk that crosses the operand's end, element by element:
@@ -602,7 +628,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   if constexpr (ST) st_e[4] = stamp_clock();
   const bool st_wrote =
 #endif
-  finish_unit<OUTT, D, NWD, OROW, 32, WBUF / 2>(p, mbase, b, hk, unit, split, R, tid);
+  finish_unit<OUTT, D, NWD, OROW, 32, WBUF / 2, RB>(p, mbase, b, hk, unit, split, R, tid, row0);
 #ifdef FFAI_STAMPS
   if constexpr (ST) st_e[5] = stamp_clock();
   if (st_rec) {

@@ -20,8 +20,28 @@ hipError_t launch_dec(const DecodeParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Row blocks of 16 or 32 rows (row_block), every key in one workgroup of the most waves.
+template <int MODE, int OUTT, int D, bool KT, int NWD>
+hipError_t launch_rows(const DecodeParams& p, hipStream_t s) {
+  const int rows = p.group * p.Tq;
+  const dim3 grid((unsigned)p.Hkv, (unsigned)((rows + p.row_block - 1) / p.row_block),
+                  (unsigned)p.B);
+  if (p.row_block == 16)
+    hipLaunchKernelGGL((decode_kernel<MODE, OUTT, D, KT, NWD, 1, true>), grid, dim3(NWD * 64), 0,
+                       s, p);
+  else
+    hipLaunchKernelGGL((decode_kernel<MODE, OUTT, D, KT, NWD, 2, true>), grid, dim3(NWD * 64), 0,
+                       s, p);
+  return hipGetLastError();
+}
+
 template <int MODE, int OUTT, int D, bool KT>
 hipError_t pick_waves(const DecodeParams& p, int waves, hipStream_t s) {
+  if (p.row_block) {
+    if (waves <= 4) return launch_rows<MODE, OUTT, D, KT, 4>(p, s);
+    if constexpr (D == 64) return launch_rows<MODE, OUTT, D, KT, 8>(p, s);
+    return hipErrorInvalidValue;
+  }
   if (waves == 1) return launch_dec<MODE, OUTT, D, KT, 1>(p, s);
   if (waves == 2) return launch_dec<MODE, OUTT, D, KT, 2>(p, s);
   if (waves == 4) return launch_dec<MODE, OUTT, D, KT, 4>(p, s);

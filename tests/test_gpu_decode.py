@@ -6,6 +6,8 @@ and HIP graph replays."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -313,3 +315,42 @@ def test_two_calls_share_nothing_but_the_workspace(gpu):
     e1, e2 = max_abs(_host(o1), w1), max_abs(_host(o2), w2)
     print(f"shared workspace: {e1:.3e} {e2:.3e}")
     assert e1 < TOL_BF16 and e2 < TOL_BF16
+
+
+@pytest.mark.parametrize("dtype,rnd", [(torch.bfloat16, round_bf16), (torch.float16, round_f16)])
+@pytest.mark.parametrize("case", [
+    # (batch, q heads, kv heads, queries, keys, head_dim, k transposed, causal, ragged, rows a block)
+    (1, 4, 4, 33, 8, 64, False, False, False, 16),        # a last block of one row, one short tile
+    (2, 3, 3, 227, 227, 64, False, True, True, 16),       # a prompt, ragged, one batch item empty
+    (1, 16, 16, 227, 1500, 64, True, False, False, 16),   # 240 blocks, 8 waves, 3 rounds of tiles
+    (1, 20, 20, 400, 450, 64, False, True, False, 0),     # 260 blocks of 32: the fused kernel
+    (1, 20, 20, 380, 449, 64, False, True, False, 32),    # 240 blocks of 32, a tail of one key
+    (2, 6, 2, 50, 324, 64, True, True, False, 16),        # groups of 3: blocks across positions
+    (1, 12, 2, 70, 1028, 128, False, True, False, 16),    # head_dim 128, 4 waves
+    (1, 24, 4, 180, 452, 128, True, False, True, 32),
+])
+def test_row_blocks(gpu, case, dtype, rnd):
+    """Short grids of more rows than a unit holds run as row blocks on the decode kernel, with f32
+    and same-type output, K and V rows past a ragged length filled with inf and NaN."""
+    b, hq, hkv, tq, tk, d, kt, causal, ragged, block = case
+    rng = np.random.default_rng(tq * 1000 + tk)
+    q, k, v = (rnd(randn(rng, s)) for s in ((b, hq, tq, d), (b, hkv, tk, d), (b, hkv, tk, d)))
+    lens = np.array([0, tk - 5][-b:], np.int32) if ragged else None
+    off = tk - tq if causal else 0
+    want = oracle.attend_general(q, k, v, k_transposed=False, scale=d ** -0.5, causal=causal,
+                                 q_offset=off, kv_lens=lens)
+    if ragged:
+        for i, n in enumerate(lens):
+            k[i, :, n:], v[i, :, n:] = np.inf, np.nan
+    qd, vd = _dev(q, dtype, gpu), _dev(v, dtype, gpu)
+    kd = _dev(np.ascontiguousarray(np.swapaxes(k, 2, 3)) if kt else k, dtype, gpu)
+    kw = dict(scale=d ** -0.5, causal=causal, q_offset=off, k_transposed=kt,
+              kv_lens=None if lens is None else torch.from_numpy(lens).to(gpu))
+    for out_dtype in (torch.float32, dtype):
+        out = torch.full((b, hq, tq, d), float("nan"), dtype=out_dtype, device=gpu)
+        desc = fa.make_desc(qd, kd, vd, out, **kw)
+        assert L.load().ffai_attn_row_block(ctypes.byref(desc)) == block
+        fa.attention(qd, kd, vd, out=out, **kw)
+        err = max_abs(_host(out), want)
+        print(f"row blocks {case} {dtype} out {out_dtype}: {err:.3e}")
+        assert err < TOL_BF16
