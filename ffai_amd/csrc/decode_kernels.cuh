@@ -291,11 +291,10 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   // `valid`: the tile's keys before the end of the cache (wave-uniform). Blocks of K or V rows
   // that hold none of them are not read: their LDS rows keep stale values, whose keys are masked
   // and whose V rows are cleared once the DMA has landed (ragged tails of per-beam caches).
-  auto dma_tile = [&](int it, int valid) {
+  auto dma_k = [&](int it, int valid) {
     const int64_t kb = (int64_t)it * BN;
-    const uint32_t kla = lds_addr(kl), vla = lds_addr(vl);
+    const uint32_t kla = lds_addr(kl);
     const char* kbase = reinterpret_cast<const char*>(kp + (KT ? kb : kb * p.k_st));
-    const char* vbase = reinterpret_cast<const char*>(vp + kb * p.v_st);
 #pragma unroll
     for (int j = 0; j < KBUF / 512; ++j) {
       const int r = j * KRB + kr;
@@ -303,6 +302,11 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
           (uint32_t)(2 * (r * p.k_st + 8 * (KT ? swz_kt(r, kpc) : swz_kr(r, kpc))));
       if (KT || j * KRB < valid) lds_dma16_sbase<!RB>(kbase, off, kla + j * 1024);
     }
+  };
+  auto dma_v = [&](int it, int valid) {
+    const int64_t kb = (int64_t)it * BN;
+    const uint32_t vla = lds_addr(vl);
+    const char* vbase = reinterpret_cast<const char*>(vp + kb * p.v_st);
 #pragma unroll
     for (int j = 0; j < VBUF / 512; ++j) {
       const int r = j * VRB + vr;
@@ -315,12 +319,12 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   // last valid key read that key's row instead; K^T 8-key chunks that would cross the
   // operand's end read the tile's first chunk. The slots of masked keys then hold finite
   // stand-ins; the valid keys of the one K^T chunk that crosses the end are patched afterwards.
-  auto dma_tile_clamped = [&](int it) {
+  auto dma_k_clamped = [&](int it) {
     const int kb = it * BN;
     const int klast = kv_end - 1;
-    const uint32_t kla = lds_addr(kl), vla = lds_addr(vl);
+    const uint32_t kla = lds_addr(kl);
     const char* kbase = reinterpret_cast<const char*>(kp + (KT ? kb : (int64_t)kb * p.k_st));
-    const char* vbase = reinterpret_cast<const char*>(vp + (int64_t)kb * p.v_st);
+    (void)klast;
 #pragma unroll
     for (int j = 0; j < KBUF / 512; ++j) {
       const int r = j * KRB + kr;
@@ -335,6 +339,12 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
         lds_dma16_sbase<!RB>(kbase, off, kla + j * 1024);
       }
     }
+  };
+  auto dma_v_clamped = [&](int it) {
+    const int kb = it * BN;
+    const int klast = kv_end - 1;
+    const uint32_t vla = lds_addr(vl);
+    const char* vbase = reinterpret_cast<const char*>(vp + (int64_t)kb * p.v_st);
 #pragma unroll
     for (int j = 0; j < VBUF / 512; ++j) {
       const int r = j * VRB + vr;
@@ -444,11 +454,45 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   // Issue tile `it`'s loads (by DMA, or through registers for a short end).
   auto issue_tile = [&](int it) {
     const int kb = it * BN;
-    if (kb + BN <= kv_end || tail_dma_of(kb)) dma_tile(it, min(BN, kv_end - kb));
-    else if (end_dma_of(kb)) dma_tile_clamped(it);
-    else stage_tile(it);
+    if (kb + BN <= kv_end || tail_dma_of(kb)) {
+      dma_k(it, min(BN, kv_end - kb));
+      dma_v(it, min(BN, kv_end - kb));
+    } else if (end_dma_of(kb)) {
+      dma_k_clamped(it);
+      dma_v_clamped(it);
+    } else {
+      stage_tile(it);
+    }
     if (patch_end_of(kb)) patch_kt_load();
   };
+  // AHEAD: a wave's next tile is loaded under the current one, its K into the K region once the
+  // current scores have read theirs, its V into the V region once the current output has (a
+  // second region per wave would not fit in LDS). For row blocks at head_dim 128, whose four
+  // waves are one to a SIMD: 16 heads x 64 rows x 3072 keys 28.8 -> 24.7 us, 3 heads x 1200 causal
+  // 15.4 -> 14.3. At head_dim 64 the other wave of the SIMD covers the loads already (16 heads x
+  // 227 rows x 1500 keys 8.8 -> 9.3). DMA only: false for a short end, whose registers would be
+  // live throughout.
+  constexpr bool AHEAD = RB && D == 128;
+  auto prefetch_k = [&](int it) {
+    const int kb = it * BN;
+    if (kb + BN <= kv_end || tail_dma_of(kb)) dma_k(it, min(BN, kv_end - kb));
+    else if (end_dma_of(kb)) dma_k_clamped(it);
+    else return false;
+    if (patch_end_of(kb)) patch_kt_load();
+    return true;
+  };
+  auto prefetch_v = [&](int it) {
+    const int kb = it * BN;
+    if (kb + BN <= kv_end || tail_dma_of(kb)) dma_v(it, min(BN, kv_end - kb));
+    else dma_v_clamped(it);
+  };
+  // waits until at most the 16 loads issued last (a tile's K or V) are outstanding
+  static_assert(!AHEAD || (KBUF / 512 == 16 && VBUF / 512 == 16), "the waits' count");
+  auto wait_all_but_last = [&]() {
+    __builtin_amdgcn_s_waitcnt(0x4f70);  // vmcnt(16)
+    asm volatile("" ::: "memory");
+  };
+  bool ahead = false;  // the tile's loads were issued under the previous tile
 #ifdef FFAI_STAMPS
   // event times of the workgroup, recorded by wave 0 (diagnostic builds only; attn_common.cuh),
   // for head_dim 64 (the head_dim-128 instantiations keep their register budget without them)
@@ -484,14 +528,17 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
     const bool has = it < t_end;  // wave-uniform
     const int kb = it * BN;
     if (!has) continue;
-    if (i > 0) {
+    if (i > 0 && !(AHEAD && ahead)) {
       // the tile region is this wave's own: reuse needs only its own earlier LDS reads done
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
       issue_tile(it);
     }
     const bool tail_dma = tail_dma_of(kb), end_dma = end_dma_of(kb);
     const bool patch_end = patch_end_of(kb);
-    vm_wait_all();
+    // a whole tile loaded ahead: its K has landed once only its V loads, issued after, may be out
+    const bool v_out = AHEAD && ahead && kb + BN <= kv_end;
+    if (v_out) wait_all_but_last();
+    else vm_wait_all();
 #ifdef FFAI_STAMPS
     if (ST && i == 0) st_e[2] = stamp_clock();
 #endif
@@ -525,6 +572,14 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
         }
 #pragma unroll
         for (int c = 0; c < NC; ++c) sacc[c][kb4] = mfma16x16<MODE>(a, qf[c][h], sacc[c][kb4]);
+      }
+    }
+    if constexpr (AHEAD) {
+      // this tile's K reads are done: the next tile's K
+      ahead = false;
+      if (it + NWD < t_end) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        ahead = prefetch_k(it + NWD);
       }
     }
     // ---- mask (only tiles that reach past a row's last visible key: the ragged end, or the
@@ -583,6 +638,13 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
 #pragma unroll
         for (int db = 0; db < D / 16; ++db) oacc[c][db] *= corr[c];
     }
+    if constexpr (AHEAD) {
+      // this tile's V has landed once only the next tile's K loads may be out
+      if (v_out) {
+        if (ahead && kb + NWD * BN + BN <= kv_end) wait_all_but_last();
+        else vm_wait_all();
+      }
+    }
     // ---- O^T += V^T P^T: A(d = 16 db + n16, slot e) = V(key of slot e, d), read transposed from
     //      the [key][d] tile: rows r and r + 16 share the chunk permutation
 #pragma unroll
@@ -596,6 +658,12 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) oacc[c][db] = mfma16x16<MODE>(a, pf[c][ch], oacc[c][db]);
       }
+    if constexpr (AHEAD) {
+      if (ahead) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this tile's V reads are done
+        prefetch_v(it + NWD);
+      }
+    }
   }
 
   // ---- merge the waves' partials through LDS (the tile area is free once all waves pass here)
