@@ -224,51 +224,66 @@ struct CrossParams {
   int64_t src_rs;
   int32_t t, heads, head_dim, n_tblk;
   int32_t src_vec;
+  int32_t grid;  // workgroups of each of K and V
 };
 
-// V (and K in rows layout): output row (h, t) = input row t, columns h*D .. h*D + D - 1.
-template <int SRC, int DST>
-__global__ __launch_bounds__(256) void cross_rows_kernel(const void* src, void* dst, CrossParams p) {
-  const int row_units = p.heads * p.head_dim / 8;
-  const int64_t units = (int64_t)p.t * row_units;
-  const auto* s = reinterpret_cast<const store_t<SRC>*>(src);
-  auto* o = reinterpret_cast<store_t<DST>*>(dst);
-  for (int64_t u = (int64_t)wg_id_x() * 256 + item_id(); u < units; u += (int64_t)gridDim.x * 256) {
-    const int t = (int)(u / row_units);
-    const int col = (int)(u - (int64_t)t * row_units) * 8;
-    const int h = col / p.head_dim, d = col - h * p.head_dim;
-    float x[8];
-    load8<SRC>(s + (int64_t)t * p.src_rs + col, p.src_vec, x);
-    store8<DST>(o + ((int64_t)h * p.t + t) * p.head_dim + d, true, x);
-  }
-}
-
+// The whole build in one launch: blockIdx.y 0 is V, 1 is K.
+// V, and K in rows layout: output row (h, t) = input row t, columns h*D .. h*D + D - 1.
 // K^T: output (h, d, t). Workgroup (head h, 64-frame block): the block's 64 x head_dim values go
-// through LDS so that both the reads (along d) and the writes (along t) are contiguous.
-template <int SRC, int DST>
-__global__ __launch_bounds__(256) void cross_kt_kernel(CrossParams p) {
-  __shared__ float tile[64][128 + 1];
-  const int tb = wg_id_x() % p.n_tblk, h = wg_id_x() / p.n_tblk;
-  const int t0 = tb * 64;
-  const int rows = min(64, p.t - t0);
+// through LDS so that both the reads (along d) and the writes (along t) are contiguous, 8 frames
+// a store at whatever alignment the row (t elements long) has.
+// One launch for both, since the caller's launches bound the build, not its traffic (a layer's
+// 18 MB, 1500 frames x 16 heads, move in ~4 us): 24 layers, eager, rows layout, in two launches a
+// layer 319 us, so 240; 12 layers of 733 frames x 8 heads 159 and 119.
+template <int SRC, int DST, bool KT>
+__global__ __launch_bounds__(256) void cross_build_kernel(CrossParams p) {
+  __shared__ float tile[KT ? 64 : 1][128 + 1];
+  if (!KT || wg_id_y() == 0) {
+    const int row_units = p.heads * p.head_dim / 8;
+    const int64_t units = (int64_t)p.t * row_units;
+    const auto* s = reinterpret_cast<const store_t<SRC>*>(wg_id_y() == 0 ? p.sv : p.sk);
+    auto* o = reinterpret_cast<store_t<DST>*>(wg_id_y() == 0 ? p.v : p.k);
+    for (int64_t u = (int64_t)wg_id_x() * 256 + item_id(); u < units; u += (int64_t)p.grid * 256) {
+      const int t = (int)(u / row_units);
+      const int col = (int)(u - (int64_t)t * row_units) * 8;
+      const int h = col / p.head_dim, d = col - h * p.head_dim;
+      float x[8];
+      load8<SRC>(s + (int64_t)t * p.src_rs + col, p.src_vec, x);
+      store8<DST>(o + ((int64_t)h * p.t + t) * p.head_dim + d, true, x);
+    }
+    return;
+  }
   const int du = p.head_dim / 8;
   const auto* s = reinterpret_cast<const store_t<SRC>*>(p.sk);
-  for (int u = item_id(); u < rows * du; u += 256) {
-    const int r = u / du, d = (u - r * du) * 8;
-    float x[8];
-    load8<SRC>(s + (int64_t)(t0 + r) * p.src_rs + h * p.head_dim + d, p.src_vec, x);
+  for (int blk = wg_id_x(); blk < p.heads * p.n_tblk; blk += p.grid) {
+    const int tb = blk % p.n_tblk, h = blk / p.n_tblk;
+    const int t0 = tb * 64;
+    const int rows = min(64, p.t - t0);
+    __syncthreads();  // the previous block's reads of the tile
+    for (int u = item_id(); u < rows * du; u += 256) {
+      const int r = u / du, d = (u - r * du) * 8;
+      float x[8];
+      load8<SRC>(s + (int64_t)(t0 + r) * p.src_rs + h * p.head_dim + d, p.src_vec, x);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) tile[r][d + e] = x[e];
-  }
-  __syncthreads();
-  auto* o = reinterpret_cast<store_t<DST>*>(p.k) + (int64_t)h * p.head_dim * p.t;
-  // one output element per thread and step: row d, frame t0 + c
-  for (int u = item_id(); u < p.head_dim * 64; u += 256) {
-    const int d = u / 64, c = u % 64;
-    if (c >= rows) continue;
-    const float x = tile[c][d];
-    if constexpr (DST == kF32) o[(int64_t)d * p.t + t0 + c] = x;
-    else o[(int64_t)d * p.t + t0 + c] = from_f32<DST>(x);
+      for (int e = 0; e < 8; ++e) tile[r][d + e] = x[e];
+    }
+    __syncthreads();
+    auto* o = reinterpret_cast<store_t<DST>*>(p.k) + (int64_t)h * p.head_dim * p.t + t0;
+    // row d, frames t0 + 8 c .. + 7: 8 lanes a row (and 8 rows) of a wave, no two on one LDS bank
+    for (int u = item_id(); u < p.head_dim * 8; u += 256) {
+      const int d = u >> 3, c = (u & 7) * 8;
+      auto* row = o + (int64_t)d * p.t + c;
+      if (c + 8 <= rows) {
+        st4<DST>(row, f32x4{tile[c][d], tile[c + 1][d], tile[c + 2][d], tile[c + 3][d]});
+        st4<DST>(row + 4, f32x4{tile[c + 4][d], tile[c + 5][d], tile[c + 6][d], tile[c + 7][d]});
+      } else {
+        for (int e = 0; c + e < rows; ++e) {
+          const float x = tile[c + e][d];
+          if constexpr (DST == kF32) row[e] = x;
+          else row[e] = from_f32<DST>(x);
+        }
+      }
+    }
   }
 }
 
@@ -312,16 +327,15 @@ struct AppendLaunch {
 };
 template <int S, int D>
 struct CrossLaunch {
-  static hipError_t run(const CrossParams& p, bool kt, hipStream_t st) {
+  static hipError_t run(CrossParams p, bool kt, hipStream_t st) {
     const int64_t units = (int64_t)p.t * p.heads * p.head_dim / 8;
-    const unsigned grid = (unsigned)std::min<int64_t>((units + 255) / 256, 4096);
-    hipLaunchKernelGGL((cross_rows_kernel<S, D>), dim3(grid), dim3(256), 0, st, p.sv, p.v, p);
-    if (kt) {
-      hipLaunchKernelGGL((cross_kt_kernel<S, D>), dim3((unsigned)(p.heads * p.n_tblk)), dim3(256), 0,
-                         st, p);
-    } else {
-      hipLaunchKernelGGL((cross_rows_kernel<S, D>), dim3(grid), dim3(256), 0, st, p.sk, p.k, p);
-    }
+    const int64_t blocks = std::max<int64_t>((units + 255) / 256, kt ? (int64_t)p.heads * p.n_tblk : 0);
+    p.grid = (int)std::min<int64_t>(blocks, 4096);
+    const dim3 grid((unsigned)p.grid, 2);
+    if (kt)
+      hipLaunchKernelGGL((cross_build_kernel<S, D, true>), grid, dim3(256), 0, st, p);
+    else
+      hipLaunchKernelGGL((cross_build_kernel<S, D, false>), grid, dim3(256), 0, st, p);
     return hipGetLastError();
   }
 };
