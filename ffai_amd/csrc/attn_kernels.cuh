@@ -13,8 +13,8 @@
 //   * With QW = 2 a wave computes two 32-query column blocks against each K/V fragment it
 //     reads from LDS, halving LDS operand traffic per FLOP (at 32 queries per wave the LDS
 //     read bandwidth alone would cap the MFMA pipes near 80 %).
-//   * K and V tiles are staged through LDS once per workgroup. f32: double-buffered, K as rows
-//     and V transposed, permuted in registers on the way in. 16-bit: three buffers filled by
+//   * K and V tiles are staged through LDS once per workgroup. f32: K as rows and V transposed,
+//     permuted in registers on the way in, or as three bf16 planes each. 16-bit: three buffers filled by
 //     global->LDS DMA in the layout they have in HBM (K^T or K rows, V rows), read back with
 //     transposing LDS reads where an operand needs the other orientation. One barrier per tile.
 //   * Online softmax in base 2 with v_exp_f32. f32 kernel: the running max only moves when a
@@ -41,7 +41,8 @@ namespace {
 // ---------------------------------------------------------------------------------------------
 // The forward kernel.
 //   MODE  kBF16 / kF16: Q, K, V are that 16-bit type; both products on 32x32x16 MFMA.
-//         kF32: Q f32, K/V of type KVT widened to f32 in LDS; both products on 32x32x2 f32 MFMA.
+//         kF32: Q f32, K/V of type KVT widened to f32 in LDS; both products on 32x32x2 f32 MFMA,
+//         or, all operands f32 and four waves, on 32x32x16 bf16 MFMA as sums of three bf16 parts.
 //   OUTT  output type. D head_dim. KT: K given transposed (d-major). NW waves per workgroup.
 //   QW    32-query column blocks per wave.
 // ---------------------------------------------------------------------------------------------
@@ -56,6 +57,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   using QS = store_t<MODE>;                            // Q global storage type
   static_assert(F32 || KVT == MODE, "16-bit kernels read Q, K and V of one type");
   static_assert(!F32 || QW == 1, "the f32 kernel uses one column block per wave");
+  // f32 operands as sums of three bf16 parts on the bf16 MFMA (see split_loop below).
+  constexpr bool SPL = F32 && KVT == kF32 && NW == 4;
   // LDS tiles.
   //   f32:    K [key][d] (KROW = D + 4), V^T [d][key] (VROW = BN + 4) - transposed on the way in;
   //           rows padded so that the 128-bit stores and the operand reads are conflict-free.
@@ -67,16 +70,18 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   constexpr int KROW = F32 ? D + 4 : D;
   constexpr int KTROW = BN;
   constexpr int VROW = F32 ? BN + 4 : D;
-  constexpr int KBUF = (!F32 && KT) ? D * KTROW : BN * KROW;
-  constexpr int VBUF = F32 ? D * VROW : BN * VROW;
+  //   SPL:    three 16-bit planes of K and of V, each laid out as the 16-bit kernels' tile (single-
+  //           buffered: 48 KB, two workgroups per CU).
+  constexpr int KBUF = SPL ? 3 * BN * D / 2 : (!F32 && KT) ? D * KTROW : BN * KROW;
+  constexpr int VBUF = SPL ? 3 * BN * D / 2 : F32 ? D * VROW : BN * VROW;
   // f32: double-buffered, one barrier per tile at the tile's end. 16-bit: the next tile is
   // staged and published (barrier) before the current tile's last product, so that product
   // overlaps the next tile's first one. Tile i's K is last read before the barrier of tile i,
   // its V after it (the last product): when that barrier stages tile i + 2, K(i + 2) can take
   // K(i)'s buffer but V(i + 2) needs a third. Head_dim 128 keeps two K buffers (80 KB of LDS:
   // two workgroups per CU); head_dim 64 keeps three of each (48 KB, as measured).
-  constexpr int NBUF = F32 ? 2 : 3;                    // V buffers
-  constexpr int NBK = F32 ? 2 : (D == 128 ? 2 : 3);  // K buffers
+  constexpr int NBUF = SPL ? 1 : F32 ? 2 : 3;                    // V buffers
+  constexpr int NBK = SPL ? 1 : F32 ? 2 : (D == 128 ? 2 : 3);  // K buffers
   __shared__ __attribute__((aligned(16))) LT k_lds[NBK * KBUF];
   __shared__ __attribute__((aligned(16))) LT v_lds[NBUF * VBUF];
 
@@ -137,7 +142,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   constexpr int BM = NW * 32 * QW;
   const int q0 = qb * BM + wave * 32 * QW;  // this wave's first query row
 #ifdef FFAI_STAMPS
-  const int64_t st_rec = (p.stamps && hw < p.stamp_wgs) ? ((int64_t)hw * NW + wave) * 32 : -1;
+  const int64_t st_rec = (!F32 && p.stamps && hw < p.stamp_wgs) ? ((int64_t)hw * NW + wave) * 32 : -1;
   auto stamp_now = [&](int k, uint64_t v) {
     if (st_rec >= 0 && lane == 0) stamp_put(p.stamps, st_rec + k, v);
   };
@@ -165,6 +170,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   // ---- Q fragments (B operand of S^T = K Q^T), resident for the whole key loop
   constexpr int QF = F32 ? D / 2 : D / 16;
   std::conditional_t<F32, float, u32x4> qf[QW][QF];
+  auto load_q = [&]() {
 #pragma unroll
   for (int c = 0; c < QW; ++c) {
     const int row = q0 + 32 * c + n32;
@@ -187,6 +193,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
       }
     }
   }
+  };
+  if constexpr (!SPL) load_q();
 
   // ---- staging: global -> registers (two tiles ahead) -> LDS
   // f32:    K rows -> units of 4 elements; K^T -> 4 d-rows x 4 keys (transposed in registers);
@@ -421,6 +429,61 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
     }
   };
 
+  // SPL: the same registers as load_tile, from scalar bases and one 32-bit lane offset each (the
+  // host keeps a tile's rows within 2^31 bytes of its first): 64-bit lane addresses live through
+  // the loop would spill. Tails as there, but a K^T row's end as one load moved into place.
+  auto load_split = [&](int it) {
+    if constexpr (SPL) {
+      const int kb = __builtin_amdgcn_readfirstlane(it) * BN;
+      const int klast = kv_end - 1;
+      const bool full = kb + BN <= kv_end;
+      const int64_t ks = p.k_st, vs = p.v_st;
+      auto at = [](const char* base, uint32_t off) {
+        return *reinterpret_cast<const f32x4_e*>(base + off);
+      };
+      if constexpr (KT) {
+        const int d4 = tid / (BN / 4), k4 = tid % (BN / 4);
+        // keys past the row's end: whichever the row has (masked, whatever they are)
+        const int key0 = kb + 4 * k4, s0 = full ? key0 : max(0, min(key0, p.Tk - 4));
+        const int sh = key0 - s0, kbase = full ? kb : 0;  // (a tail's s0 may lie before the tile)
+        const uint32_t off = (uint32_t)(4 * (4 * d4 * (int)ks + (s0 - kbase)));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          f32x4 x;
+          if (full || p.Tk >= 4) {
+            x = at(kp_dma + 4 * ((int64_t)kbase + r * ks), off);
+          } else {
+            const KVS* row = kp + (4 * d4 + r) * ks;  // kb is 0
+            x = f32x4{row[0], row[min(1, p.Tk - 1)], row[min(2, p.Tk - 1)], 0.f};
+          }
+          if (!full) {
+            if (sh & 1) x = f32x4{x[1], x[2], x[3], x[3]};
+            if (sh & 2) x = f32x4{x[2], x[3], x[3], x[3]};
+          }
+          kreg[r] = x;
+        }
+      } else {
+        const int k0 = tid / (D / 4), c = tid % (D / 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = k0 + i * (NT / (D / 4));  // in the tile
+          const int kc = full ? key : min(key, klast - kb);
+          kreg[i] = at(kp_dma + 4 * (int64_t)kb * ks, (uint32_t)(4 * (kc * (int)ks + 4 * c)));
+        }
+      }
+      const int k4 = tid / (D / 4), d4 = tid % (D / 4);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if (full) {
+          vreg[r] = at(vp_dma + 4 * ((int64_t)kb + r) * vs, (uint32_t)(4 * (4 * k4 * (int)vs + 4 * d4)));
+        } else {
+          const int kc = min(4 * k4 + r, klast - kb);
+          vreg[r] = at(vp_dma + 4 * (int64_t)kb * vs, (uint32_t)(4 * (kc * (int)vs + 4 * d4)));
+        }
+      }
+    }
+  };
+
   // ---- online-softmax state, per column block: this lane's query row, its half of the keys
   f32x16 oacc[QW][D / 32];
 #pragma unroll
@@ -439,7 +502,9 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   const float sl2 = p.scale_log2;
 
   if (t_begin < t_end) {
-    if constexpr (F32) {
+    if constexpr (SPL) {
+      load_split(t_begin);
+    } else if constexpr (F32) {
       load_tile(t_begin);
       store_tile(0, 0, t_begin);
       if (t_begin + 1 < t_end) load_tile(t_begin + 1);
@@ -470,14 +535,41 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
     }
   };
 
-  if constexpr (F32) {
-    // ---------------------------------------------------------------------------------------
-    // f32: both products on 32x32x2 f32 MFMA (MFMA-bound by a wide margin; no interleaving).
-    // ---------------------------------------------------------------------------------------
-    for (int it = t_begin; it < t_end; ++it) {
-      const int buf = (it - t_begin) & 1;
-      const LT* kl = k_lds + buf * KBUF;
-      const LT* vl = v_lds + buf * VBUF;
+  // f32: mask, online softmax of tile `kb`'s scores (the weights replace them), rescale of O.
+  auto softmax_f32 = [&](f32x16 (&sacc)[QW][2], int kb) {
+    if (kb + BN > kv_end || (p.causal && kb + BN - 1 > p.q_offset + q0)) {
+      mask_subtile(sacc, kb, 0);
+      mask_subtile(sacc, kb, 1);
+    }
+    float mx = kNegInf;
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(sacc[0][st][r], sacc[0][st][r + 1]));
+    const float mx_s = partner_max(mx) * sl2;
+    if (__builtin_amdgcn_ballot_w64(mx_s > m_s[0] + kRescaleSlack) != 0) {
+      const float m_new = fmaxf(m_s[0], mx_s);
+      const float corr = fast_exp2(m_s[0] - ((m_new == kNegInf) ? 0.f : m_new));
+      m_s[0] = m_new;
+      l_run[0] *= corr;
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt) oacc[0][dt] *= corr;
+    }
+    const float mc = (m_s[0] == kNegInf) ? 0.f : m_s[0];
+    float rs = 0.f;
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float e = fast_exp2(__builtin_fmaf(sacc[0][st][r], sl2, -mc));
+        sacc[0][st][r] = e;
+        rs += e;
+      }
+    l_run[0] += rs;
+  };
+  // f32: one tile's two products on 32x32x2 f32 MFMA, from f32 LDS tiles and Q in qf.
+  auto f32_tile = [&](const LT* kl, const LT* vl, int kb) {
+    if constexpr (F32) {
       f32x16 sacc[QW][2];
 #pragma unroll
       for (int st = 0; st < 2; ++st)
@@ -492,36 +584,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
 #pragma unroll
           for (int e = 0; e < 4; ++e) sacc[0][st] = mfma_f32(a[e], qf[0][4 * j + e], sacc[0][st]);
         }
-      const int kb = it * BN;
-      if (kb + BN > kv_end || (p.causal && kb + BN - 1 > p.q_offset + q0)) {
-        mask_subtile(sacc, kb, 0);
-        mask_subtile(sacc, kb, 1);
-      }
-      float mx = kNegInf;
-#pragma unroll
-      for (int st = 0; st < 2; ++st)
-#pragma unroll
-        for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(sacc[0][st][r], sacc[0][st][r + 1]));
-      const float mx_s = partner_max(mx) * sl2;
-      if (__builtin_amdgcn_ballot_w64(mx_s > m_s[0] + kRescaleSlack) != 0) {
-        const float m_new = fmaxf(m_s[0], mx_s);
-        const float corr = fast_exp2(m_s[0] - ((m_new == kNegInf) ? 0.f : m_new));
-        m_s[0] = m_new;
-        l_run[0] *= corr;
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt) oacc[0][dt] *= corr;
-      }
-      const float mc = (m_s[0] == kNegInf) ? 0.f : m_s[0];
-      float rs = 0.f;
-#pragma unroll
-      for (int st = 0; st < 2; ++st)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float e = fast_exp2(__builtin_fmaf(sacc[0][st][r], sl2, -mc));
-          sacc[0][st][r] = e;
-          rs += e;
-        }
-      l_run[0] += rs;
+      softmax_f32(sacc, kb);
 #pragma unroll
       for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
@@ -534,6 +597,231 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
             for (int e = 0; e < 4; ++e)
               oacc[0][dt] = mfma_f32(a[e], sacc[0][st][4 * j + e], oacc[0][dt]);
           }
+    }
+  };
+
+  if constexpr (SPL) {
+    // ---------------------------------------------------------------------------------------
+    // f32 products on the bf16 MFMA, 16 times the f32 MFMA's rate: every operand is the sum of
+    // three bf16 parts (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1); the differences
+    // are exact, and the three parts hold all 24 bits), and a product is the six part products of
+    // weight 2^-18 and above, smallest first, each exact and summed in f32; the three left out are
+    // below 2^-26 of it. K and V tiles are split once per workgroup on the way into LDS (three
+    // planes in the 16-bit kernels' layout), Q once per wave, the weights in registers.
+    // An element that is infinite, or so large that its first part would be, or tiny, has no such
+    // parts: a workgroup that meets one starts over on the f32 MFMA.
+    // Six bf16 products take 6/16 of the f32 MFMA's time, which bounded the kernel; now the
+    // splitting's VALU work beside them does as much. Launches, f32 MFMA and this: 6 heads x 1500
+    // 53.6 -> 35.9 us, 16 heads x 1037 71.4 -> 43.2, 8 x 12 heads x 1500 600 -> 330 (92 and 167
+    // TFLOP/s). Error against 64 bits at those sizes 4.1e-7 and 3.3e-7 (the f32 MFMA rounds its
+    // sum after every second product, this one after every sixteenth).
+    // ---------------------------------------------------------------------------------------
+    constexpr int PL = BN * D;  // elements of a plane
+    constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
+    __shared__ int f32_only;  // some element has no parts
+    uint16_t* kpl = reinterpret_cast<uint16_t*>(k_lds);
+    uint16_t* vpl = reinterpret_cast<uint16_t*>(v_lds);
+    // two elements to a packed pair of each part
+    auto split2 = [](float x, float y, uint32_t (&w)[3]) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        w[k] = pack2<kBF16>(x, y);
+        if (k < 2) {
+          x -= to_f32<kBF16>(w[k] & 0xffffu);
+          y -= __uint_as_float(w[k] & 0xffff0000u);
+        }
+      }
+    };
+    // An element is left to the f32 MFMA when its first part would overflow (from kSplitMax up), or
+    // when the largest of its group of four (of one key, or of one column of V) is below 2^-100:
+    // the MFMA takes parts below 2^-126 as zero, which there would show.
+    constexpr uint32_t kSplitMax = 0x7f7f7fffu, kSplitMin = 0x0d800000u;
+    // the bits of a group's largest magnitude to the running extremes (zero groups count as large)
+    uint32_t ext_hi = 0u, ext_lo = 0xffffffffu;
+    auto extremes = [&](float a, float b, float c, float d) {
+      const uint32_t m = __float_as_uint(fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d))));
+      ext_hi = max(ext_hi, m);
+      ext_lo = min(ext_lo, m - 1u);
+    };
+    auto no_parts = [&]() { return ext_hi > kSplitMax || ext_lo < kSplitMin; };
+    // Split the tile `it` held in kreg / vreg into the LDS planes (V rows past the last valid key
+    // zeroed); true if some element has no parts.
+    auto store_planes = [&](int it) -> bool {
+      const int kb = it * BN, klast = kv_end - 1;
+      const bool full = kb + BN <= kv_end;
+      auto put = [&](uint16_t* dst, f32x4 x) {
+        uint32_t lo[3], hi[3];
+        split2(x[0], x[1], lo);
+        split2(x[2], x[3], hi);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x2*>(dst + k * PL) = u32x2{lo[k], hi[k]};
+      };
+      ext_hi = 0u;
+      ext_lo = 0xffffffffu;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (KT) {
+          const int r = 4 * (tid / (BN / 4)) + i, c = tid % (BN / 4);
+          put(&kpl[r * BN + 8 * swz_kt(r, c >> 1) + 4 * (c & 1)], kreg[i]);
+          extremes(kreg[0][i], kreg[1][i], kreg[2][i], kreg[3][i]);
+        } else {
+          const int u = tid + i * NT, r = u / (D / 4), c = u % (D / 4);
+          put(&kpl[r * D + 8 * swz_kr(r, c >> 1) + 4 * (c & 1)], kreg[i]);
+          extremes(kreg[i][0], kreg[i][1], kreg[i][2], kreg[i][3]);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * (tid / (D / 4)) + i, c = tid % (D / 4);
+        if (!full && kb + r > klast) vreg[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        put(&vpl[r * D + 8 * swz_v(r, c >> 1) + 4 * (c & 1)], vreg[i]);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) extremes(vreg[0][e], vreg[1][e], vreg[2][e], vreg[3][e]);
+      return no_parts();
+    };
+    // Q: step s, lane group g: d = 16 s + 8 g .. +7 of the lane's row
+    u32x4 qs[3][D / 16];
+    bool q_big = false;
+    {
+      const int row = q0 + n32;
+      const float* qr = qp + (int64_t)min(row, p.Tq - 1) * p.q_st;
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) {
+        uint32_t w[4][3];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          f32x4 x = ld4f<kF32>(qr + 16 * s + 8 * g + 4 * k);
+          if (row >= p.Tq) x = f32x4{0.f, 0.f, 0.f, 0.f};
+          extremes(x[0], x[1], x[2], x[3]);
+          split2(x[0], x[1], w[2 * k]);
+          split2(x[2], x[3], w[2 * k + 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) qs[k][s] = u32x4{w[0][k], w[1][k], w[2][k], w[3][k]};
+      }
+      q_big = __builtin_amdgcn_ballot_w64(no_parts()) != 0;
+    }
+    // transposing reads, as in the 16-bit kernels below
+    const int jt = lane & 15;
+    const int tr_row = jt >> 2, tr_col = 4 * (jt & 3);
+    const int half16 = 16 * ((lane >> 4) & 1);
+    auto kfrag = [&](const uint16_t* kl, int st, int s) -> u32x4 {
+      if constexpr (KT) {
+        const int r = 16 * s + 8 * g + tr_row;
+        const int col = 32 * st + half16 + tr_col;
+        const uint16_t* base = &kl[r * BN + 8 * swz_kt(r, col >> 3) + (col & 7)];
+        const u32x2 lo = lds_tr(base), hi = lds_tr(base + 4 * BN);
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+      } else {
+        const int r = 32 * st + n32;
+        return ld16(&kl[r * D + 8 * swz_kr(r, 2 * s + g)]);
+      }
+    };
+    auto vfrag = [&](const uint16_t* vl, int t, int dt) -> u32x4 {
+      const int r = 16 * t + 4 * g + tr_row;
+      const int col = 32 * dt + half16 + tr_col;
+      const uint16_t* base = &vl[r * D + 8 * swz_v(r, col >> 3) + (col & 7)];
+      const u32x2 a0 = lds_tr(base), a1 = lds_tr(base + 8 * D);
+      return u32x4{a0.x, a0.y, a1.x, a1.y};
+    };
+    if (tid == 0) f32_only = 0;
+    __syncthreads();
+    bool redo = false;
+    for (int it = t_begin; it < t_end; ++it) {
+      const int kb = it * BN;
+      // (every wave has finished with the previous tile's planes: the barrier at the loop's end)
+      if (store_planes(it) || q_big) f32_only = 1;
+      __syncthreads();
+      redo = __builtin_amdgcn_readfirstlane(f32_only) != 0;  // the same for every wave
+      if (redo) break;
+      f32x16 sacc[QW][2];
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sacc[0][st][r] = 0.f;
+      // each step's fragments are read under the previous step's products
+      u32x4 a[2][2][3];
+      auto read_k = [&](int s) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) a[s & 1][st][k] = kfrag(kpl + k * PL, st, s);
+      };
+      read_k(0);
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) {
+        __builtin_amdgcn_sched_barrier(0);  // (steps run into each other spill)
+        if (s + 1 < D / 16) read_k(s + 1);
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+          for (int st = 0; st < 2; ++st)
+            sacc[0][st] = mfma16<kBF16>(a[s & 1][st][PA[i]], qs[PB[i]][s], sacc[0][st]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // the next tile's registers, under the softmax and the second product
+      if (it + 1 < t_end) load_split(it + 1);
+      auto read_v = [&](int t) {
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) a[t & 1][dt][k] = vfrag(vpl + k * PL, t, dt);
+      };
+      softmax_f32(sacc, kb);
+      // parts of the weights of keys 16 t + 4 g + e (e < 4) and 16 t + 8 + 4 g + e - 4, as they lie
+      u32x4 pf[2][3];
+      auto split_p = [&](int t) {
+        uint32_t w[4][3];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          split2(sacc[0][t >> 1][8 * (t & 1) + 2 * k], sacc[0][t >> 1][8 * (t & 1) + 2 * k + 1],
+                 w[k]);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) pf[t & 1][k] = u32x4{w[0][k], w[1][k], w[2][k], w[3][k]};
+      };
+      read_v(0);
+      split_p(0);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (t < 3) {
+          read_v(t + 1);
+          split_p(t + 1);
+        }
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt)
+            oacc[0][dt] = mfma16<kBF16>(a[t & 1][dt][PA[i]], pf[t & 1][PB[i]], oacc[0][dt]);
+      }
+      __syncthreads();
+    }
+    if (redo) {
+      m_s[0] = kNegInf;
+      l_run[0] = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[0][dt][r] = 0.f;
+      load_q();
+#pragma unroll 1
+      for (int it = t_begin; it < t_end; ++it) {
+        load_split(it);
+        __syncthreads();
+        store_tile(0, 0, it);
+        __syncthreads();
+        f32_tile(k_lds, v_lds, it * BN);
+      }
+      __syncthreads();
+    }
+  } else if constexpr (F32) {
+    // ---------------------------------------------------------------------------------------
+    // f32 on the f32 MFMA (one-wave launches and 16-bit K/V).
+    // ---------------------------------------------------------------------------------------
+    for (int it = t_begin; it < t_end; ++it) {
+      const int buf = (it - t_begin) & 1;
+      f32_tile(k_lds + buf * KBUF, v_lds + buf * VBUF, it * BN);
       if (it + 1 < t_end) {
         store_tile(buf ^ 1, buf ^ 1, it + 1);
         if (it + 2 < t_end) load_tile(it + 2);

@@ -1,0 +1,97 @@
+"""The four-wave f32 kernel's products, each f32 operand the sum of three bf16 parts: errors at the
+level of f32 sums over magnitudes from 2^-112 to 2^112, tile and row remainders in both K layouts, and
+operands without such parts (infinite, within half a bf16 step of overflow, or tiny)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from ffai_amd import flash_attn as fa
+from tests.helpers import randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(gpu, q, k, v, k_transposed, scale):
+    kd = np.ascontiguousarray(np.swapaxes(k, 2, 3)) if k_transposed else k
+    # (a fresh tensor: an axis of one key may carry any stride in numpy)
+    q, kd, v = (torch.empty(x.shape, device=gpu).copy_(torch.from_numpy(x)) for x in (q, kd, v))
+    out = torch.empty(q.shape, device=gpu)
+    assert fa.plan(q, kd, v, out, k_transposed=k_transposed, scale=scale)["shape"] == "wave4"
+    assert fa.attention(q, kd, v, k_transposed=k_transposed, scale=scale, out=out) is not None
+    return out.cpu().numpy().astype(np.float64)
+
+
+def _exact(q, k, v, scale):
+    q, k, v = (x.astype(np.float64) for x in (q, k, v))
+    s = np.matmul(q, np.swapaxes(k, 2, 3)) * scale
+    w = np.exp(s - s.max(-1, keepdims=True))
+    return np.matmul(w / w.sum(-1, keepdims=True), v)
+
+
+@pytest.mark.parametrize("k_transposed", [True, False])
+@pytest.mark.parametrize("queries,keys", [(33, 1), (33, 3), (64, 63), (129, 64), (100, 65),
+                                          (128, 127), (257, 1037), (64, 4098)])
+def test_remainders(gpu, queries, keys, k_transposed):
+    """Relative error in the 2-norm at most 1e-6: scores of 64 products (sqrt(64) / 2 steps of 2^-24
+    of a score of ~1, so ~2.4e-7 of a weight), as many again from v_exp_f32 and the weighted sum."""
+    rng = np.random.default_rng(queries * 5000 + keys)
+    q, k, v = (randn(rng, (2, 3, n, 64)) for n in (queries, keys, keys))
+    want = _exact(q, k, v, 0.125)
+    got = _run(gpu, q, k, v, k_transposed, 0.125)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"{queries} x {keys} kt={k_transposed}: {err:.2e}")
+    assert err < 1e-6
+
+
+@pytest.mark.parametrize("e", [-100, -60, -20, 20, 60, 100])
+def test_magnitudes(gpu, e):
+    """Keys and values 2^e times wider (queries 2^-e), and values spread over 2^+-12 within a row:
+    parts are relative to each element, so no magnitude loses bits (below 2^-100, where the third
+    part would underflow, on the f32 MFMA)."""
+    rng = np.random.default_rng(600 + e)
+    q, k, v = (randn(rng, (1, 2, n, 64)) for n in (96, 200, 200))
+    v *= np.exp2(rng.integers(-12, 13, size=v.shape)).astype(np.float32)
+    q, k, v = np.ldexp(q, -e), np.ldexp(k, e), np.ldexp(v, e)
+    want = _exact(q, k, v, 0.125)
+    got = _run(gpu, q, k, v, True, 0.125)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"2^{e}: {err:.2e}")
+    assert err < 1e-6
+
+
+@pytest.mark.parametrize("k_transposed", [True, False])
+def test_infinite_and_largest_elements(gpu, k_transposed):
+    """An infinite value reaches its column only, values near the largest f32 stay finite, and keys
+    at -inf score -inf and weigh nothing, in the first tile, a later one and the tail."""
+    rng = np.random.default_rng(620)
+    q, k, v = (randn(rng, (1, 3, n, 64)) for n in (130, 200, 200))
+    q[..., 5] = np.abs(q[..., 5]) + 0.1
+    gone = [3, 100, 199]
+    k[0, 0, gone, 5] = -np.inf          # head 0: three keys at -inf
+    v[0, 1, 70, 9] = np.inf             # head 1: column 9 infinite
+    v[0, 2, 198, 11] = 3.4e38           # head 2: column 11 huge
+    kept = [j for j in range(200) if j not in gone]
+    got = _run(gpu, q, k, v, k_transposed, 0.125)
+    want0 = _exact(q[:, :1], k[:, :1, kept], v[:, :1, kept], 0.125)
+    assert np.linalg.norm(got[:, :1] - want0) / np.linalg.norm(want0) < 1e-6
+    cols = [d for d in range(64) if d != 9]
+    want1 = _exact(q[:, 1:2], k[:, 1:2], v[:, 1:2][..., cols], 0.125)
+    assert np.all(np.isposinf(got[:, 1, :, 9]))
+    assert np.linalg.norm(got[:, 1:2][..., cols] - want1) / np.linalg.norm(want1) < 1e-6
+    want2 = _exact(q[:, 2:], k[:, 2:], v[:, 2:], 0.125)
+    err = np.abs(got[:, 2:] - want2) / np.abs(want2).max((2,), keepdims=True)
+    assert err.max() < 4e-6
+
+
+def test_a_tiny_column_beside_others(gpu):
+    """A column of V at 2^-118 beside columns at 1 keeps its own relative precision."""
+    rng = np.random.default_rng(640)
+    q, k, v = (randn(rng, (1, 2, n, 64)) for n in (70, 150, 150))
+    v[0, 1, :, 20] = np.ldexp(v[0, 1, :, 20], -118)
+    want = _exact(q, k, v, 0.125)
+    got = _run(gpu, q, k, v, False, 0.125)
+    err = np.linalg.norm(got - want, axis=2) / np.linalg.norm(want, axis=2)
+    assert err.max() < 1.2e-6
