@@ -43,14 +43,23 @@ namespace {
 //   MODE  kBF16 / kF16: Q, K, V are that 16-bit type; both products on 32x32x16 MFMA.
 //         kF32: Q f32, K/V of type KVT widened to f32 in LDS; both products on 32x32x2 f32 MFMA,
 //         or, all operands f32 and four waves, on 32x32x16 bf16 MFMA as sums of three bf16 parts.
-//   OUTT  output type. D head_dim. KT: K given transposed (d-major). NW waves per workgroup.
+//   OUTT  output type. D head_dim. KT: K given transposed (d-major). WAVES per workgroup.
 //   QW    32-query column blocks per wave.
+//   WAVES 8: two key groups of four waves, the second on the second half of the work's keys
+//         through its own tile ring; the first merges the two in LDS. For grids of at most one
+//         workgroup per CU, which otherwise leave one wave to a SIMD and nothing to cover its
+//         chain of LDS, product and exp latencies; a second workgroup's worth of key pieces
+//         instead pays their merge through memory. 20 heads x 1500 frames (240 items) bf16: 28.6
+//         us with one group, 26.9 in 2 pieces, 23.6 so; 12 heads 26.5 and 21.3; 20 heads x 800
+//         16.6 and 14.2; 6 heads x 1500 in 3 pieces (216 workgroups) 16.2 and 14.9.
 // ---------------------------------------------------------------------------------------------
 // Four-wave launches are built for two workgroups per CU (<= 256 VGPRs): the second wave on each
 // SIMD is what hides the first one's exp and dependency latencies.
-template <int MODE, int KVT, int OUTT, int D, bool KT, int NW, int QW>
-__global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2 : 1) void fwd_kernel(FwdParams p) {
-  constexpr int NT = NW * 64;
+template <int MODE, int KVT, int OUTT, int D, bool KT, int WAVES, int QW>
+__global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32)) ? 2 : 1) void fwd_kernel(FwdParams p) {
+  constexpr int KS = WAVES == 8 ? 2 : 1;  // key groups
+  constexpr int NW = WAVES / KS;          // waves of a key group
+  constexpr int NT = NW * 64;  // threads of a key group
   constexpr bool F32 = (MODE == kF32);
   using LT = std::conditional_t<F32, float, uint16_t>;  // LDS / compute storage type
   using KVS = store_t<KVT>;                            // K/V global storage type
@@ -82,8 +91,9 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   // two workgroups per CU); head_dim 64 keeps three of each (48 KB, as measured).
   constexpr int NBUF = SPL ? 1 : F32 ? 2 : 3;                    // V buffers
   constexpr int NBK = SPL ? 1 : F32 ? 2 : (D == 128 ? 2 : 3);  // K buffers
-  __shared__ __attribute__((aligned(16))) LT k_lds[NBK * KBUF];
-  __shared__ __attribute__((aligned(16))) LT v_lds[NBUF * VBUF];
+  static_assert(KS == 1 || (KS == 2 && !F32 && QW == 1), "two key groups: 16-bit, 32 rows a wave");
+  __shared__ __attribute__((aligned(16))) LT k_lds_all[KS * NBK * KBUF];
+  __shared__ __attribute__((aligned(16))) LT v_lds_all[KS * NBUF * VBUF];
 
   // ---- which work (an item, or one piece of a split item) this workgroup computes
   const int hw = wg_id_x();
@@ -134,7 +144,11 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   const int b = bh / p.Hq;
   const int hk = h / (p.Hq / p.Hkv);
 
-  const int tid = item_id();
+  // key group, and the thread and wave within it
+  const int grp = KS > 1 ? __builtin_amdgcn_readfirstlane(item_id() / NT) : 0;
+  const int tid = KS > 1 ? item_id() % NT : item_id();
+  LT* const k_lds = k_lds_all + grp * (NBK * KBUF);
+  LT* const v_lds = v_lds_all + grp * (NBUF * VBUF);
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: keeps q0 scalar
   const int g = lane >> 5;    // lane group: which half of each MFMA contraction step
@@ -142,7 +156,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   constexpr int BM = NW * 32 * QW;
   const int q0 = qb * BM + wave * 32 * QW;  // this wave's first query row
 #ifdef FFAI_STAMPS
-  const int64_t st_rec = (!F32 && p.stamps && hw < p.stamp_wgs) ? ((int64_t)hw * NW + wave) * 32 : -1;
+  const int64_t st_rec = (!F32 && grp == 0 && p.stamps && hw < p.stamp_wgs) ? ((int64_t)hw * NW + wave) * 32 : -1;
   auto stamp_now = [&](int k, uint64_t v) {
     if (st_rec >= 0 && lane == 0) stamp_put(p.stamps, st_rec + k, v);
   };
@@ -157,8 +171,11 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
   if (p.causal) kv_blk = min(kv_end, max(0, p.q_offset + min(qb * BM + BM, p.Tq)));
   const int n_tiles = (kv_blk + BN - 1) / BN;
   const int tps = split < 0 ? n_tiles : (n_tiles + p.n_split - 1) / p.n_split;
-  const int t_begin = split < 0 ? 0 : split * tps;
-  const int t_end = min(n_tiles, t_begin + tps);
+  const int w_begin = split < 0 ? 0 : split * tps;  // the work's tiles
+  const int w_end = min(n_tiles, w_begin + tps);
+  const int half = KS > 1 ? (max(0, w_end - w_begin) + 1) / 2 : 0;
+  const int t_begin = w_begin + grp * half;  // and this key group's
+  const int t_end = KS > 1 && grp == 0 ? w_begin + half : w_end;
 
   const QS* qp = reinterpret_cast<const QS*>(p.q) + b * p.q_sb + h * p.q_sh;
   const KVS* kp = reinterpret_cast<const KVS*>(p.k) + b * p.k_sb + hk * p.k_sh;
@@ -1228,6 +1245,41 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && (D == 64 || MODE != kF32)) ? 2
 #endif
   }
 
+  if constexpr (KS > 1) {
+    // one barrier a tile: the second group may have a tile fewer
+    if (max(0, t_end - t_begin) < half) __syncthreads();
+    __syncthreads();  // every wave has finished with the tiles
+    // the second group's partials to LDS, lane-major (thread t merges what thread NT + t wrote)
+    f32x4* mo = reinterpret_cast<f32x4*>(k_lds_all);
+    f32x2* ml = reinterpret_cast<f32x2*>(v_lds_all);
+    static_assert(KS * NBK * KBUF * sizeof(LT) >= NT * D / 8 * sizeof(f32x4), "the O partials fit");
+    if (grp == 1) {
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          mo[(4 * dt + r) * NT + tid] = f32x4{oacc[0][dt][4 * r], oacc[0][dt][4 * r + 1],
+                                              oacc[0][dt][4 * r + 2], oacc[0][dt][4 * r + 3]};
+      ml[tid] = f32x2{m_s[0], l_run[0]};
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const f32x2 o_ml = ml[tid];
+    const float m_new = fmaxf(m_s[0], o_ml[0]);
+    const float mc = (m_new == kNegInf) ? 0.f : m_new;  // both empty: weights 0, not NaN
+    const float c0 = fast_exp2(m_s[0] - mc), c1 = fast_exp2(o_ml[0] - mc);
+    m_s[0] = m_new;
+    l_run[0] = l_run[0] * c0 + o_ml[1] * c1;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const f32x4 x = mo[(4 * dt + r) * NT + tid];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          oacc[0][dt][4 * r + e] = oacc[0][dt][4 * r + e] * c0 + x[e] * c1;
+      }
+  }
 #ifdef FFAI_STAMPS
   // exit times (recording workgroups, lane 0)
   auto stamp_exit = [&]() {

@@ -371,3 +371,34 @@ def test_broad_seeded_sweep_against_the_oracle(gpu, split_override):
         assert _counters_zero(ws), (case, plan)
     print("kernels", kernels, "worst", {t: f"{e:.2e}" for t, e in worst.items()})
     assert set(kernels) == {"fwd", "decode"}
+
+
+@pytest.mark.parametrize("dtype,rnd", [(torch.bfloat16, round_bf16), (torch.float16, round_f16)])
+@pytest.mark.parametrize("h,tq,tk,causal,kt,pieces", [
+    (20, 300, 65, False, False, 1),    # two tiles: one a key group, the second a single key
+    (6, 1500, 320, False, True, 3),    # pieces of two tiles, the last of one: its second group empty
+    (6, 1500, 1500, False, False, 3),  # pieces of 8 tiles
+    (12, 1037, 1040, False, True, 1),  # 17 tiles: 9 and 8
+    (10, 900, 900, True, False, 1),    # causal: query blocks of 2 to 15 tiles
+])
+def test_two_key_groups(gpu, split_override, h, tq, tk, causal, kt, pieces, dtype, rnd):
+    """Four-wave grids of at most one workgroup per CU: two key groups of a work, odd and even
+    tile counts, merged in LDS, whole and under key pieces; ragged lengths down to no keys."""
+    rng = np.random.default_rng(h * 10000 + tq + tk)
+    split_override(-1, pieces)
+    b = 1
+    q, k, v = (rnd(randn(rng, s)) for s in ((b, h, tq, 64), (b, h, tk, 64), (b, h, tk, 64)))
+    kd = np.ascontiguousarray(np.swapaxes(k, 2, 3)) if kt else k
+    for lens in (None, [0], [64], [tk - 3]):
+        kw = dict(scale=0.125, causal=causal, k_transposed=kt)
+        if lens is not None:
+            kw["kv_lens"] = torch.tensor(lens, dtype=torch.int32, device=gpu)
+        out, plan, ws = _run(_dev_at(q, dtype, gpu, 0), _dev_at(kd, dtype, gpu, 0),
+                             _dev_at(v, dtype, gpu, 0), out_dtype=dtype, **kw)
+        assert plan["shape"] == "wave4" and plan["workgroups"] <= 256
+        want = oracle.attend_general(q, k, v, k_transposed=False, scale=0.125, causal=causal,
+                                     kv_lens=None if lens is None else np.array(lens, np.int32))
+        err = max_abs(out.float().cpu().numpy(), want)
+        print(f"two key groups {h} x {tq} x {tk} lens {lens}: {err:.3e}")
+        assert err < TOL_BF16
+        assert _counters_zero(ws)
