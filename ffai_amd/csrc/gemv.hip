@@ -95,10 +95,12 @@ __device__ __forceinline__ float group_max(float v) {
 }
 
 // EPI 0: y[b][o] = sum. EPI 1: the q/k/v epilogue, cache elements of type CDT.
-// TL >= 0: a specialized launch shape known at compile time (tile rows 1 << TL, NW waves, one
-// pass, the first NXL dense x loads hold every beam; ROWS > 0: exactly ROWS beams); the
-// compiler then folds the index arithmetic and unrolls the waves' reduction (~0.3-0.8 us per
-// call at the decoder's shapes).
+// TL >= 0: a launch shape of one pass and tile rows 1 << TL, known at compile time (index
+// arithmetic folds, and the reduction's parts unroll); with NW, NXL and ROWS > 0 also its waves,
+// the dense x loads that hold every beam, and the exact number of beams (the reduction's waves
+// unroll too). us per call in graphs at 5 beams, every value from the parameters / TL / all:
+// 768 x 768 3.86 / 3.24 / -, 768 x 3072 6.24 / 5.25 / -, 1024 x 1024 4.0 / 3.3 / 2.9; 5120 x 1280
+// at 8 beams 9.53 / 7.31 / -.
 // TL < 0: the shape comes from the parameters.
 template <int NJ, int EPI, int CDT, int TL = -1, int NW = 0, int NXL = 0, int ROWS = 0>
 __global__ __launch_bounds__(1024) void gemv_f16_kernel(GemvParams p, QkvCacheParams qp) {
@@ -112,7 +114,7 @@ __global__ __launch_bounds__(1024) void gemv_f16_kernel(GemvParams p, QkvCachePa
   const int tid = item_id(), lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tl = SPEC ? TL : p.tr_log2, tr = 1 << tl, qn = 16 >> tl;
-  const int nw = SPEC ? NW : p.nw;
+  const int nw = NW > 0 ? NW : p.nw;
   const int kp = nw * KW;  // one part's elements per pass
   const int m = lane & 15, g = lane >> 4;
   const int q = m >> tl, r = m & (tr - 1);  // A row m: weight row r of part q
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(1024) void gemv_f16_kernel(GemvParams p, QkvCachePa
     };
 #pragma unroll
     for (int i = 0; i < NX1; ++i) {
-      if (SPEC && i >= NXL) break;
+      if (NXL > 0 && i >= NXL) break;
       load_x(i);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -161,7 +163,7 @@ __global__ __launch_bounds__(1024) void gemv_f16_kernel(GemvParams p, QkvCachePa
       if constexpr (NX1 < NI) {
         if (i + NX1 < NI) load_x(i + NX1);
       }
-      if (SPEC ? i >= NXL : i >= ni) {  // wave-uniform
+      if (NXL > 0 ? i >= NXL : i >= ni) {  // wave-uniform
         if constexpr (NX1 < NI) continue;  // (a loop of 16 with a load would not unroll on break)
         else break;
       }
@@ -234,20 +236,30 @@ __global__ __launch_bounds__(1024) void gemv_f16_kernel(GemvParams p, QkvCachePa
     const int b = t >> tl, rr = t & (tr - 1);  // beam b, tile row rr
     const int o = tile * tr + rr;
     if (o >= p.out_dim) continue;
-    float v = 0.f;
-    for (int qq = 0; qq < qn; ++qq) {
-      const int mm = (qq << tl) + rr, nn = (qq << tl) + b;
-      const int l = nn + 16 * (mm >> 2), e = mm & 3;
-      // all the waves' values first (independent LDS reads), then the sum in wave order
-      float pv[16];
+    // all the waves' values of a part first (independent LDS reads, M >= the waves of them), then
+    // their sum in wave order
+    auto sum_waves = [&](auto m_tag) {
+      constexpr int M = decltype(m_tag)::value;
+      float v = 0.f;
 #pragma unroll
-      for (int ww = 0; ww < 16; ++ww)
-        pv[ww] = ww < nw ? reinterpret_cast<const float*>(
-                               gemv_lds + ww * reg)[4 * l + e + 16 * (l >> 4)]
-                         : 0.f;
+      for (int qq = 0; qq < qn; ++qq) {
+        const int mm = (qq << tl) + rr, nn = (qq << tl) + b;
+        const int l = nn + 16 * (mm >> 2), e = mm & 3;
+        float pv[M];
 #pragma unroll
-      for (int ww = 0; ww < 16; ++ww) v += pv[ww];
-    }
+        for (int ww = 0; ww < M; ++ww)
+          pv[ww] = reinterpret_cast<const float*>(
+              gemv_lds + min(ww, nw - 1) * reg)[4 * l + e + 16 * (l >> 4)];
+#pragma unroll
+        for (int ww = 0; ww < M; ++ww) v += ww < nw ? pv[ww] : 0.f;
+      }
+      return v;
+    };
+    float v;
+    if constexpr (NW > 0) v = sum_waves(std::integral_constant<int, NW>{});
+    else if (nw <= 4) v = sum_waves(std::integral_constant<int, 4>{});
+    else if (nw <= 8) v = sum_waves(std::integral_constant<int, 8>{});
+    else v = sum_waves(std::integral_constant<int, 16>{});
     if constexpr (EPI == 0) {
       p.y[b * p.ys + o] = v;
     } else {
@@ -271,24 +283,36 @@ __global__ __launch_bounds__(1024) void gemv_f16_kernel(GemvParams p, QkvCachePa
   }
 }
 
-// Launch shape for (out_dim, in_dim, rows): the largest tile (<= 16 rows, >= rows) that still
-// gives ~192 workgroups, then per part the fewest passes with at most 16 waves, 32 NJ elements
-// each (NJ 2, 4 or 8; 1 for a single block), NJ halved while the waves' LDS regions would exceed
-// the CU's 160 KB.
+// Launch shape for (out_dim, in_dim, rows): the largest tile (4 to 16 rows, >= rows) that still
+// gives ~192 workgroups, or 144 while a wave's part stays at two blocks; then per part the fewest
+// passes with at most 16 waves, 32 NJ elements each (NJ 2, 4 or 8; 1 for a single block), NJ
+// halved while the waves' LDS regions would exceed the CU's 160 KB.
+// us per call in graphs, 192 and 144 as the bound: 2304 x 768 at 5 beams 4.04 and 3.52 (8- and
+// 16-row tiles), 1152 x 384 greedy 2.84 and 2.52, 1280 x 1280 greedy 3.67 and 3.45; but with four
+// blocks and more the smaller tiles stream better: 1280 x 5120 greedy 7.15 and 8.81. At 128 or
+// less 1024 x 1024 greedy loses (2.46 and 3.03). Two-row tiles (384 x 384 greedy) took 3.19
+// against 2.34 with four rows: eight parts to sum at the end.
 struct GemvShape {
   int tr_log2, nw, nj, passes;
   size_t lds;
 };
+// 32-element blocks of a K part, and a wave's share of them
+int gemv_blocks(int in_dim, int tl) { return (in_dim / 8 + 4 * (16 >> tl) - 1) / (4 * (16 >> tl)); }
+int gemv_nj(int bpp) { return bpp == 1 ? 1 : (bpp + 1) / 2 <= 16 ? 2 : (bpp + 3) / 4 <= 16 ? 4 : 8; }
 GemvShape gemv_shape(int out_dim, int in_dim, int rows) {
-  int min_tl = 0;
+  int min_tl = 2;
   while ((1 << min_tl) < rows) ++min_tl;
   int tl = 4;
-  while (tl > min_tl && (out_dim + (1 << tl) - 1) / (1 << tl) < 192) --tl;
+  auto few = [&](int t) {
+    const int wgs = (out_dim + (1 << t) - 1) >> t;
+    return wgs < 144 || (wgs < 192 && gemv_nj(gemv_blocks(in_dim, t)) > 2);
+  };
+  while (tl > min_tl && few(tl)) --tl;
   const int qn = 16 >> tl;
-  const int bpp = (in_dim / 8 + 4 * qn - 1) / (4 * qn);  // 32-element blocks per part
+  const int bpp = gemv_blocks(in_dim, tl);
   GemvShape s{};
   s.tr_log2 = tl;
-  s.nj = bpp == 1 ? 1 : (bpp + 1) / 2 <= 16 ? 2 : (bpp + 3) / 4 <= 16 ? 4 : 8;
+  s.nj = gemv_nj(bpp);
   for (;;) {
     s.nw = std::min(16, (bpp + s.nj - 1) / s.nj);
     s.passes = (bpp + s.nw * s.nj - 1) / (s.nw * s.nj);
@@ -365,6 +389,17 @@ hipError_t launch_gemv(GemvParams p, const QkvCacheParams& qp, int out_rows, hip
       return e;
   }
   const dim3 block(64 * s.nw);
+  // every other single-pass shape of two or four blocks a wave: tile rows fixed
+  if (s.passes == 1 && s.nj == 2) {
+    if (s.tr_log2 == 4) return launch_one<2, EPI, CDT, 4>(s.lds, grid, block, st, p, qp);
+    if (s.tr_log2 == 3) return launch_one<2, EPI, CDT, 3>(s.lds, grid, block, st, p, qp);
+    if (s.tr_log2 == 2) return launch_one<2, EPI, CDT, 2>(s.lds, grid, block, st, p, qp);
+  }
+  if (s.passes == 1 && s.nj == 4) {
+    if (s.tr_log2 == 4) return launch_one<4, EPI, CDT, 4>(s.lds, grid, block, st, p, qp);
+    if (s.tr_log2 == 3) return launch_one<4, EPI, CDT, 3>(s.lds, grid, block, st, p, qp);
+    if (s.tr_log2 == 2) return launch_one<4, EPI, CDT, 2>(s.lds, grid, block, st, p, qp);
+  }
   if (s.nj == 1) return launch_one<1, EPI, CDT>(s.lds, grid, block, st, p, qp);
   if (s.nj == 2) return launch_one<2, EPI, CDT>(s.lds, grid, block, st, p, qp);
   if (s.nj == 4) return launch_one<4, EPI, CDT>(s.lds, grid, block, st, p, qp);

@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from oracle import gemv as og
+from ffai_amd import _lib as L
 from ffai_amd.gemv import F16Gemv, Int8Vocab
 
 pytestmark = pytest.mark.gpu
@@ -189,6 +190,24 @@ SPECIALIZED = [(1024, 1024, 5), (1024, 1024, 6), (1024, 1024, 7), (1024, 1024, 8
 @pytest.mark.parametrize("out_dim,in_dim,rows", SPECIALIZED)
 def test_gemv_f16_launch_shapes(gpu, out_dim, in_dim, rows):
     rng = np.random.default_rng(out_dim + 3 * in_dim + rows)
+    w16 = rng.standard_normal((out_dim, in_dim)).astype(np.float16)
+    x = rng.standard_normal((rows, in_dim)).astype(np.float32)
+    got = F16Gemv(torch.from_numpy(w16).to(gpu))(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    _check_f16(got, w16, x)
+
+
+@pytest.mark.parametrize("out_dim,in_dim,rows,shape", [
+    # (tile rows, blocks a wave, passes): every instance with its tile rows fixed, ragged in and out
+    (571, 520, 3, (4, 2, 1)), (575, 4104, 2, (4, 4, 1)),
+    (1151, 776, 5, (8, 2, 1)), (767, 3080, 5, (8, 4, 1)),
+    (2303, 776, 4, (16, 2, 1)), (3100, 1288, 11, (16, 4, 1)),
+    # either side of the 144 tiles from which a short part takes the taller tile
+    (1144, 384, 1, (4, 2, 1)), (1152, 384, 1, (8, 2, 1)), (1280, 5120, 1, (4, 4, 1)),
+])
+def test_gemv_f16_fixed_tile_rows(gpu, out_dim, in_dim, rows, shape):
+    p = L.gemv_plan_info(out_dim, in_dim, rows)
+    assert (p["tile_rows"], p["blocks_per_wave"], p["passes"]) == shape
+    rng = np.random.default_rng(out_dim + rows)
     w16 = rng.standard_normal((out_dim, in_dim)).astype(np.float16)
     x = rng.standard_normal((rows, in_dim)).astype(np.float32)
     got = F16Gemv(torch.from_numpy(w16).to(gpu))(torch.from_numpy(x).to(gpu)).cpu().numpy()
