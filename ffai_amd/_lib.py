@@ -58,6 +58,10 @@ class EncoderAttnWeights(ctypes.Structure):
                 for n in ("wq", "bq", "wk_scaled", "wv", "bv", "wo", "bo", "wqkv", "bqkv")]
 
 
+# split counters at the start of a workspace, the only bytes of it that must start at zero
+COUNTER_BYTES = 4096
+
+
 class TensorView(ctypes.Structure):
     _fields_ = [
         ("data", ctypes.c_void_p), ("dtype", ctypes.c_int32), ("on_device", ctypes.c_int32),
