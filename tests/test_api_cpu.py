@@ -479,3 +479,17 @@ def test_one_wave_grids_stay_within_one_round(lib):
                         if items < 384 and tk >= 128:   # room for two pieces of a tile or more
                             assert info[2] >= 2, (dt, b, heads, tq, tk, info)
     assert n > 50
+
+
+@pytest.mark.parametrize("heads,rows,keys,head_dim,splits,tiles", [
+    (6, 5, 1500, 64, 8, 3), (12, 1, 1500, 64, 8, 3), (20, 5, 1500, 64, 8, 3),
+    (6, 5, 512, 64, 1, 8),      # eight waves cover it in a round
+    (6, 5, 513, 64, 5, 2), (12, 5, 900, 64, 8, 2), (4, 6, 2048, 64, 8, 4),
+    (2, 6, 256, 128, 1, 4), (2, 6, 1024, 128, 8, 2), (2, 6, 4096, 128, 16, 4),
+    (2, 6, 16384, 64, 32, 8),   # past one round of tiles a workgroup, more pieces again
+])
+def test_decode_pieces_fit_one_merge_round(lib, heads, rows, keys, head_dim, splits, tiles):
+    """A short decode grid: at most eight pieces per unit while the workgroup's waves cover a piece
+    in one round, units of one round whole."""
+    info, _ = _plan(lib, L.BF16, L.BF16, L.F32, 1, heads, heads, rows, keys, head_dim, L.K_ROWS)
+    assert info[0] == 1 and (info[2], info[3]) == (splits, tiles)
