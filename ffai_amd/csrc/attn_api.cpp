@@ -352,7 +352,7 @@ bool plan_decode(const ffai_attn_desc* d, bool allow_split, size_t max_ws, const
 int row_block_of(const ffai_attn_desc* d, bool dma_ok) {
   const int group = d->heads_q / d->heads_kv;
   const int64_t rows = (int64_t)group * d->q_len;
-  if (d->q_dtype == FFAI_F32 || !dma_ok || rows <= 32) return 0;
+  if (d->q_dtype == FFAI_F32 || rows <= 32 || (d->head_dim == 128 && !dma_ok)) return 0;
   if (d->k_layout == FFAI_K_TRANSPOSED && d->kv_len < 4) return 0;  // 4-key chunks
   const int64_t lim = int64_t(1) << 31;  // as in plan_decode
   if (int64_t(std::max(d->head_dim, ffai::kBlockN)) * d->k_strides[2] * 2 >= lim ||
@@ -371,8 +371,8 @@ int row_block_of(const ffai_attn_desc* d, bool dma_ok) {
   return 0;
 }
 
-// `dma_ok`: f32, or K and V admit the 16-bit decode kernel's DMA (other 16-bit decode shapes take
-// fwd_kernel).
+// `dma_ok`: K and V admit the 16-bit kernels' DMA, without which the decode kernel serves head_dim
+// 64 only.
 // `max_ws`: the workspace available. Every split serves speed only, so a plan whose partials
 // would exceed it runs its split items in fewer pieces, or whole, instead.
 Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
@@ -382,7 +382,7 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
   const int64_t cus = geo.cus;
   p.cus = geo.cus;
   p.xcd_shift = std::max(0, xcd_shift_of(geo.xcds));
-  if (dma_ok && plan_decode(d, allow_split, max_ws, geo, &p)) return p;
+  if ((dma_ok || d->head_dim == 64) && plan_decode(d, allow_split, max_ws, geo, &p)) return p;
   const int64_t bh = (int64_t)d->batch * d->heads_q;
   const bool f32 = d->q_dtype == FFAI_F32;
   const int n_tiles = (d->kv_len + ffai::kBlockN - 1) / ffai::kBlockN;
@@ -536,7 +536,7 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
 // Workspace for a descriptor whatever the operands' alignment turns out to be.
 size_t plan_ws_bytes(const ffai_attn_desc* d) {
   const size_t dma = make_plan(d, true, true).ws_bytes;
-  return d->q_dtype == FFAI_F32 ? dma : std::max(dma, make_plan(d, true, false).ws_bytes);
+  return d->head_dim == 64 ? dma : std::max(dma, make_plan(d, true, false).ws_bytes);
 }
 
 // ---- allocation-free entry point: a library-owned split-key scratch per device ----------------
@@ -650,6 +650,7 @@ int run_fwd(const ffai_attn_desc* d, const void* q, const void* k, const void* v
     p.Tq = d->q_len; p.Tk = d->kv_len;
     p.causal = d->causal; p.q_offset = d->q_offset;
     p.n_split = pl.n_split; p.tiles_per_split = pl.tiles_per_split; p.n_work = pl.n_work;
+    p.dma = dma_ok;
     p.row_block = row_block;
     p.scale_log2 = d->scale * 1.4426950408889634f;
 #ifdef FFAI_STAMPS

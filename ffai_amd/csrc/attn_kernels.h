@@ -56,8 +56,7 @@ struct FwdParams {
 #endif
 };
 
-// A decode launch: at most 32 query rows (group x Tq) per (batch, kv-head) unit or row block; 16-bit: K and V
-// that admit the DMA's 16-byte row accesses (8-byte K^T rows).
+// A decode launch: at most 32 query rows (group x Tq) per (batch, kv-head) unit or row block.
 struct DecodeParams {
   const void* q;
   const void* k;
@@ -75,6 +74,7 @@ struct DecodeParams {
   int32_t n_split;          // workgroups per unit
   int32_t tiles_per_split;  // 64-key tiles per workgroup
   int32_t n_work;           // B * Hkv * n_split
+  int32_t dma;              // K and V admit the tiles' DMA (16-byte rows, K^T rows 8); 16-bit
   int32_t row_block;        // 0, or the rows (16 or 32) of a unit's row blocks: any number of
                             // query rows, n_split 1
   float scale_log2;

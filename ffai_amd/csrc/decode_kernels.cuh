@@ -273,8 +273,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   // column c0 + 4 (j % 4), and then holds column c0 + j of rows r0 .. r0 + 3
   const int tr_row = n16 >> 2, tr_col = 4 * (n16 & 3);
 
-  // ---- staging (the host launches this kernel only for operands that admit its vector
-  //      accesses). Rows of K and V: 16-byte units, the key index clamped to the last valid key
+  // ---- staging. Rows of K and V: 16-byte units, the key index clamped to the last valid key
   //      and zeroed past it. K^T rows: 4-key (8-byte) chunks, each loaded when all four keys are
   //      valid and zeroed otherwise; the one chunk per row that straddles the last valid key is
   //      then patched element by element in LDS. Every address stays inside the operand.
@@ -403,11 +402,11 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
         kreg[j] = u32x4{v0 ? lo.x : 0u, v0 ? lo.y : 0u, v1 ? hi.x : 0u, v1 ? hi.y : 0u};
       } else {
         const int key = kb + u / (D / 8), c = u % (D / 8);
-        const u32x4 x = ld16(kp + (int64_t)min(key, klast) * p.k_st + 8 * c);
+        const u32x4 x = ld16h(kp + (int64_t)min(key, klast) * p.k_st + 8 * c);
         kreg[j] = key <= klast ? x : u32x4{0u, 0u, 0u, 0u};
       }
       const int key = kb + u / (D / 8), c = u % (D / 8);
-      const u32x4 x = ld16(vp + (int64_t)min(key, klast) * p.v_st + 8 * c);
+      const u32x4 x = ld16h(vp + (int64_t)min(key, klast) * p.v_st + 8 * c);
       vreg[j] = key <= klast ? x : u32x4{0u, 0u, 0u, 0u};
     }
 #pragma unroll
@@ -446,15 +445,21 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   // anything (inf, NaN) and a masked weight of 0 times NaN is NaN: they are cleared in LDS once
   // the DMA has landed. (K^T only) the chunk that crosses the operand's end is not read whole by
   // the DMA and is patched.
-  auto tail_dma_of = [&](int kb) { return kb + BN > kv_end && kb + BN <= p.Tk; };
-  auto end_dma_of = [&](int kb) { return kb + BN > p.Tk && kb + 8 <= p.Tk; };
+  // Operands off the DMA's alignment (K^T rows of an odd length) come through registers, every tile:
+  // 16 heads x 5 rows x 1499 keys 9.0 us so (7.6 by DMA over 1500), 23.2 on the fused kernel; row
+  // blocks, 6 heads x 100 rows x 1037 keys 10.1 and 18.6, 12 heads x 257 x 257 6.4 and 12.5.
+  // (Head_dim 64 only: at 128 the choice spills scalar registers, and the host sends such operands
+  // to the fused kernel.)
+  const bool dma = D == 128 || p.dma != 0;
+  auto tail_dma_of = [&](int kb) { return dma && kb + BN > kv_end && kb + BN <= p.Tk; };
+  auto end_dma_of = [&](int kb) { return dma && kb + BN > p.Tk && kb + 8 <= p.Tk; };
   auto patch_end_of = [&](int kb) {
     return KT && end_dma_of(kb) && ((kv_end - 1) & ~7) + 8 > p.Tk;
   };
   // Issue tile `it`'s loads (by DMA, or through registers for a short end).
   auto issue_tile = [&](int it) {
     const int kb = it * BN;
-    if (kb + BN <= kv_end || tail_dma_of(kb)) {
+    if ((dma && kb + BN <= kv_end) || tail_dma_of(kb)) {
       dma_k(it, min(BN, kv_end - kb));
       dma_v(it, min(BN, kv_end - kb));
     } else if (end_dma_of(kb)) {
@@ -475,6 +480,7 @@ __global__ __launch_bounds__(NWD * 64) void decode_kernel(DecodeParams p) {
   constexpr bool AHEAD = RB && D == 128;
   auto prefetch_k = [&](int it) {
     const int kb = it * BN;
+    if (!dma) return false;
     if (kb + BN <= kv_end || tail_dma_of(kb)) dma_k(it, min(BN, kv_end - kb));
     else if (end_dma_of(kb)) dma_k_clamped(it);
     else return false;

@@ -125,21 +125,21 @@ int ffai_attn_fwd_noalloc(const ffai_attn_desc* d, const void* q, const void* k,
 size_t ffai_attn_noalloc_scratch_bytes(void);
 
 /* Diagnostic, no counterpart in the reference: the launch plan ffai_attn_fwd uses for `d` when
- * every operand admits the kernels' vector accesses (16-byte aligned bases and strides), so a
+ * K and V are 16-byte aligned (bases and strides; at head_dim 64 whatever they are), so a
  * test or benchmark can state which kernel shape it ran. info[0]: kernel (0 the fused
  * encoder/prefill kernel, 1 the decode kernel); info[1]: workgroup shape (fused: 0 one wave x
  * 32 query rows, 1 four waves x 32 rows, 2 four waves x 64 rows, 3 the same on 16x16x32 MFMA;
  * decode: waves per workgroup);
  * info[2]: key splits per work item (1 = no partials); info[3]: 64-key tiles per split;
  * info[4]: workgroups. Where ffai_attn_row_block is not 0 the call runs as row blocks instead, and
- * this is the plan it has with operands off that alignment. Returns FFAI_OK, FFAI_DECLINED or
- * FFAI_ERR_INVALID as ffai_attn_workspace_bytes. */
+ * this is the plan a forced split or launch shape would start from. Returns FFAI_OK, FFAI_DECLINED
+ * or FFAI_ERR_INVALID as ffai_attn_workspace_bytes. */
 int ffai_attn_plan_info(const ffai_attn_desc* d, int32_t info[5]);
 
-/* Diagnostic, no counterpart in the reference: whether ffai_attn_fwd (and _noalloc) runs `d`, with
- * K and V 16-byte aligned, as row blocks: a short grid of 16-bit prompt or window rows on the
- * decode kernel, one workgroup per block over all its keys, using no workspace. Returns the query
- * rows per block (16 or 32), 0 when the call runs its plan (or is declined), or
+/* Diagnostic, no counterpart in the reference: whether ffai_attn_fwd (and _noalloc) runs `d` as row
+ * blocks (at head_dim 128 with K and V 16-byte aligned): a short grid of 16-bit prompt or window
+ * rows on the decode kernel, one workgroup per block over all its keys, using no workspace.
+ * Returns the query rows per block (16 or 32), 0 when the call runs its plan (or is declined), or
  * FFAI_ERR_INVALID. */
 int ffai_attn_row_block(const ffai_attn_desc* d);
 

@@ -354,3 +354,32 @@ def test_row_blocks(gpu, case, dtype, rnd):
         err = max_abs(_host(out), want)
         print(f"row blocks {case} {dtype} out {out_dtype}: {err:.3e}")
         assert err < TOL_BF16
+
+
+@pytest.mark.parametrize("dtype,rnd", [(torch.bfloat16, round_bf16), (torch.float16, round_f16)])
+@pytest.mark.parametrize("h,tq,tk,d,kt", [
+    (6, 5, 4, 64, True), (6, 5, 37, 64, True), (12, 3, 1037, 64, True), (3, 20, 449, 64, False),
+    (2, 6, 333, 128, True), (5, 100, 65, 64, True), (16, 227, 517, 64, True),
+    (3, 100, 131, 128, True), (4, 60, 131, 128, False),
+])
+def test_operands_off_the_dma_alignment(gpu, h, tq, tk, d, kt, dtype, rnd):
+    """Every operand one element off 16-byte boundaries, K^T rows of an odd length: units and row
+    blocks staged through registers, ragged ends filled with NaN among them."""
+    rng = np.random.default_rng(tq * 2000 + tk)
+    q, k, v = (rnd(randn(rng, s)) for s in ((2, h, tq, d), (2, h, tk, d), (2, h, tk, d)))
+    lens = np.array([tk, max(1, tk - 9)], np.int32)
+    want = oracle.attend_general(q, k, v, k_transposed=False, scale=d ** -0.5, kv_lens=lens)
+    k[1, :, lens[1]:], v[1, :, lens[1]:] = np.nan, np.inf
+
+    def shifted(x):
+        flat = torch.zeros(x.size + 1, dtype=dtype, device=gpu)
+        flat[1:] = _dev(x.reshape(-1), dtype, gpu)
+        return flat[1:].view(*x.shape)
+
+    out = torch.zeros(q.size + 1, device=gpu)[1:].view(*q.shape)
+    kd = shifted(np.ascontiguousarray(np.swapaxes(k, 2, 3)) if kt else k)
+    kw = dict(scale=d ** -0.5, k_transposed=kt, kv_lens=torch.from_numpy(lens).to(gpu))
+    fa.attention(shifted(q), kd, shifted(v), out=out, **kw)
+    err = max_abs(_host(out), want)
+    print(f"off alignment {h} x {tq} x {tk} d{d} kt{int(kt)} {dtype}: {err:.3e}")
+    assert err < TOL_BF16
