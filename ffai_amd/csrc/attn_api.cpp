@@ -428,11 +428,12 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
   // items than CUs take up to three, so that about every CU holds a piece: whisper-tiny (6
   // heads, 72 items) bf16 17.1 us in 3 pieces against 26.3 whole (6: 17.0); a whisper-large-v3
   // window (20 heads, 240 items) runs whole: 27.4 us against 26.6 in 2 and 27.4 in 3. f32
-  // four-wave grids (two workgroups per CU) of fewer items than CUs fill the 512 slots:
-  // whisper-tiny f32 50.5 us in 6 pieces against 56.4 in 3, 66.2 in 4 (288 works: a second
-  // round) and 77.9 in 2; up to 1024 items they aim at ~4096 waves (300 items: 183 us in 4
-  // pieces against 236 whole, 197 in 2, 211 in 8). One-wave 16-bit grids (prompt steps,
-  // misaligned decode) fill at most the 768 slots of three workgroups per CU (48 KB of LDS
+  // four-wave grids (two workgroups per CU) of fewer items than CUs fill the 512 slots: 6 heads x
+  // 1500 36.5 us in 6 pieces against 40.0 in 5, 44.8 in 4 (288 works: a second round), 41.1 in 3,
+  // 53.7 in 2 and 91 whole; 16 heads x 1037 44.0 in 3, 55.1 in 4, 56.5 in 2; up to 1024 items they
+  // aim at ~4096 waves (300 items, when the f32 MFMA bounded them: 183 us in 4 pieces against 236
+  // whole, 197 in 2, 211 in 8). One-wave 16-bit grids (prompt steps
+  // past row_block_of's limits, head_dim-128 decode off the DMA's alignment) fill at most the 768 slots of three workgroups per CU (48 KB of LDS
   // each): the cross-attention of 228 tokens, 128 items, 14.6 us in 6 pieces against 15.4 in 5,
   // 15.7 in 4 and 19.2 in 7 (896 workgroups: a second round). One-wave f32 grids (two per CU)
   // keep about 512 workgroups: f32 decode over 1500 keys, 6 heads: 25.9 us in 24 pieces, 32.7
