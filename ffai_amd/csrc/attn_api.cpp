@@ -412,9 +412,11 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
     p.variant = forced == ffai::kWave4x2x16 ? ffai::kWave4x2 : forced;
     p.x16 = forced == ffai::kWave4x2x16;
   }
-  // the f32 four-wave kernel addresses a tile's rows by 32-bit byte offsets from its first
+  // the f32 four-wave kernel addresses a tile's rows (the last tile's K^T rows: whole ones) by 32-bit
+  // byte offsets from its first
+  const int64_t row = d->k_layout == FFAI_K_TRANSPOSED ? d->kv_len : 0;
   if (f32 && p.variant == ffai::kWave4 &&
-      (int64_t(ffai::kBlockN) * d->k_strides[2] * 4 >= (int64_t(1) << 31) ||
+      ((int64_t(ffai::kBlockN) * d->k_strides[2] + row) * 4 >= (int64_t(1) << 31) ||
        int64_t(ffai::kBlockN) * d->v_strides[2] * 4 >= (int64_t(1) << 31)))
     p.variant = ffai::kWave1;
   const int64_t items = work_of(p.variant);

@@ -460,24 +460,34 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
       };
       if constexpr (KT) {
         const int d4 = tid / (BN / 4), k4 = tid % (BN / 4);
-        // keys past the row's end: whichever the row has (masked, whatever they are)
-        const int key0 = kb + 4 * k4, s0 = full ? key0 : max(0, min(key0, p.Tk - 4));
-        const int sh = key0 - s0, kbase = full ? kb : 0;  // (a tail's s0 may lie before the tile)
-        const uint32_t off = (uint32_t)(4 * (4 * d4 * (int)ks + (s0 - kbase)));
+        if (full) {
+          const uint32_t off = (uint32_t)(4 * (4 * d4 * (int)ks + 4 * k4));
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          f32x4 x;
-          if (full || p.Tk >= 4) {
-            x = at(kp_dma + 4 * ((int64_t)kbase + r * ks), off);
-          } else {
-            const KVS* row = kp + (4 * d4 + r) * ks;  // kb is 0
-            x = f32x4{row[0], row[min(1, p.Tk - 1)], row[min(2, p.Tk - 1)], 0.f};
+          for (int r = 0; r < 4; ++r) kreg[r] = at(kp_dma + 4 * ((int64_t)kb + r * ks), off);
+        } else {
+          // keys past the last valid one: an address the row has (which may lie before the tile),
+          // and 1 (what a masked key holds must not choose the loop below)
+          const int key0 = kb + 4 * k4, s0 = max(0, min(key0, p.Tk - 4)), sh = key0 - s0;
+          uint32_t off = (uint32_t)(4 * (4 * d4 * (int)ks + s0));
+#pragma unroll
+          for (int r = 0; r < 4; ++r, off += 4u * (uint32_t)ks) {
+            if (kb + p.Tk >= 4) {
+              kreg[r] = at(kp_dma, off);
+            } else {  // (the row's start: s0 is 0)
+              auto one = [&](int e) {
+                return *reinterpret_cast<const float*>(kp_dma + (off + 4u * (uint32_t)min(e, klast - kb)));
+              };
+              kreg[r] = f32x4{one(0), one(1), one(2), 0.f};
+            }
           }
-          if (!full) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            f32x4 x = kreg[r];
             if (sh & 1) x = f32x4{x[1], x[2], x[3], x[3]};
             if (sh & 2) x = f32x4{x[2], x[3], x[3], x[3]};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kreg[r][e] = key0 + e <= klast ? x[e] : 1.f;
           }
-          kreg[r] = x;
         }
       } else {
         const int k0 = tid / (D / 4), c = tid % (D / 4);

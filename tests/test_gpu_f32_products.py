@@ -1,6 +1,7 @@
 """The four-wave f32 kernel's products, each f32 operand the sum of three bf16 parts: errors at the
-level of f32 sums over magnitudes from 2^-112 to 2^112, tile and row remainders in both K layouts, and
-operands without such parts (infinite, within half a bf16 step of overflow, or tiny)."""
+level of f32 sums over magnitudes from 2^-112 to 2^112, tile and row remainders in both K layouts,
+operands without such parts (infinite, within half a bf16 step of overflow, or tiny), and masked
+keys of any value."""
 
 from __future__ import annotations
 
@@ -14,13 +15,14 @@ from tests.helpers import randn
 pytestmark = pytest.mark.gpu
 
 
-def _run(gpu, q, k, v, k_transposed, scale):
+def _run(gpu, q, k, v, k_transposed, scale, **kw):
     kd = np.ascontiguousarray(np.swapaxes(k, 2, 3)) if k_transposed else k
     # (a fresh tensor: an axis of one key may carry any stride in numpy)
     q, kd, v = (torch.empty(x.shape, device=gpu).copy_(torch.from_numpy(x)) for x in (q, kd, v))
     out = torch.empty(q.shape, device=gpu)
-    assert fa.plan(q, kd, v, out, k_transposed=k_transposed, scale=scale)["shape"] == "wave4"
-    assert fa.attention(q, kd, v, k_transposed=k_transposed, scale=scale, out=out) is not None
+    kw.update(k_transposed=k_transposed, scale=scale)
+    assert fa.plan(q, kd, v, out, **kw)["shape"] == "wave4"
+    assert fa.attention(q, kd, v, out=out, **kw) is not None
     return out.cpu().numpy().astype(np.float64)
 
 
@@ -95,3 +97,20 @@ def test_a_tiny_column_beside_others(gpu):
     got = _run(gpu, q, k, v, False, 0.125)
     err = np.linalg.norm(got - want, axis=2) / np.linalg.norm(want, axis=2)
     assert err.max() < 1.2e-6
+
+
+@pytest.mark.parametrize("k_transposed", [True, False])
+@pytest.mark.parametrize("lens", [1, 62, 130, 190])
+def test_masked_keys_change_nothing(gpu, lens, k_transposed):
+    """Keys and values past a window's length, whatever they hold (infinite, huge, tiny, subnormal),
+    leave every bit of the result as zeros there do."""
+    rng = np.random.default_rng(690 + lens)
+    q, k, v = (randn(rng, (1, 2, n, 64)) for n in (70, 201, 201))
+    n = torch.tensor([lens], dtype=torch.int32, device=gpu)
+    k[:, :, lens:], v[:, :, lens:] = 0.0, 0.0
+    want = _run(gpu, q, k, v, k_transposed, 0.125, kv_lens=n)
+    assert np.linalg.norm(want - _exact(q, k[:, :, :lens], v[:, :, :lens], 0.125)) / \
+        np.linalg.norm(want) < 1e-6
+    for x in (np.inf, 3e38, 1e-30, 1e-40):
+        k[:, :, lens:], v[:, :, lens:] = x, x
+        assert np.array_equal(_run(gpu, q, k, v, k_transposed, 0.125, kv_lens=n), want), x
