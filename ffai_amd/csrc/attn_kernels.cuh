@@ -66,7 +66,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
   using QS = store_t<MODE>;                            // Q global storage type
   static_assert(F32 || KVT == MODE, "16-bit kernels read Q, K and V of one type");
   static_assert(!F32 || QW == 1, "the f32 kernel uses one column block per wave");
-  // f32 operands as sums of three bf16 parts on the bf16 MFMA (see split_loop below).
+  // f32 operands as sums of three bf16 parts on the bf16 MFMA (see the SPL key loop below).
   constexpr bool SPL = F32 && KVT == kF32 && NW == 4;
   // LDS tiles.
   //   f32:    K [key][d] (KROW = D + 4), V^T [d][key] (VROW = BN + 4) - transposed on the way in;
@@ -189,27 +189,27 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
   std::conditional_t<F32, float, u32x4> qf[QW][QF];
   auto load_q = [&]() {
 #pragma unroll
-  for (int c = 0; c < QW; ++c) {
-    const int row = q0 + 32 * c + n32;
-    const bool ok = row < p.Tq;
-    const QS* qr = qp + (int64_t)min(row, p.Tq - 1) * p.q_st;
-    if constexpr (F32) {
-      // step (j, e): lane group g supplies d = 8j + 4g + e
+    for (int c = 0; c < QW; ++c) {
+      const int row = q0 + 32 * c + n32;
+      const bool ok = row < p.Tq;
+      const QS* qr = qp + (int64_t)min(row, p.Tq - 1) * p.q_st;
+      if constexpr (F32) {
+        // step (j, e): lane group g supplies d = 8j + 4g + e
 #pragma unroll
-      for (int j = 0; j < D / 8; ++j) {
-        const f32x4 x = ld4f<kF32>(qr + 8 * j + 4 * g);
+        for (int j = 0; j < D / 8; ++j) {
+          const f32x4 x = ld4f<kF32>(qr + 8 * j + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) qf[c][4 * j + e] = ok ? x[e] : 0.f;
-      }
-    } else {
-      // step s: lane group g supplies d = 16s + 8g .. +7
+          for (int e = 0; e < 4; ++e) qf[c][4 * j + e] = ok ? x[e] : 0.f;
+        }
+      } else {
+        // step s: lane group g supplies d = 16s + 8g .. +7
 #pragma unroll
-      for (int s = 0; s < D / 16; ++s) {
-        const u32x4 x = ld16h(qr + 16 * s + 8 * g);
-        qf[c][s] = ok ? x : u32x4{0u, 0u, 0u, 0u};
+        for (int s = 0; s < D / 16; ++s) {
+          const u32x4 x = ld16h(qr + 16 * s + 8 * g);
+          qf[c][s] = ok ? x : u32x4{0u, 0u, 0u, 0u};
+        }
       }
     }
-  }
   };
   if constexpr (!SPL) load_q();
 
@@ -632,11 +632,16 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
     // f32 products on the bf16 MFMA, 16 times the f32 MFMA's rate: every operand is the sum of
     // three bf16 parts (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1); the differences
     // are exact, and the three parts hold all 24 bits), and a product is the six part products of
-    // weight 2^-18 and above, smallest first, each exact and summed in f32; the three left out are
-    // below 2^-26 of it. K and V tiles are split once per workgroup on the way into LDS (three
+    // weight 2^-18 and above, smallest first, each exact and summed in f32. The three left out are
+    // at most about 2^-24 of it, half a step of an f32 product: rounding to bf16 leaves |x1| <= 2^-8
+    // |x| and |x2| <= 2^-17 |x|, so x1 y2 + x2 y1 reaches 2 * 2^-25 (2^-24.2 in 4 million random
+    // pairs, 2^-27.5 rms). K and V tiles are split once per workgroup on the way into LDS (three
     // planes in the 16-bit kernels' layout), Q once per wave, the weights in registers.
-    // An element that is infinite, or so large that its first part would be, or tiny, has no such
-    // parts: a workgroup that meets one starts over on the f32 MFMA.
+    // The MFMA takes 16-bit parts below 2^-126 as zero, so an element has three parts from 2^-103
+    // up. A workgroup that meets a nonzero element below kSplitMin, or one above kSplitMax (whose
+    // part products could pass f32's range with either sign), starts over on the f32 MFMA: 8 x 12
+    // heads x 1500 547 us if all meet one in their first tile and 842 in their last, 333 in none
+    // (578 when the f32 MFMA did all; 6 heads 51, 66, 35 and 50).
     // Six bf16 products take 6/16 of the f32 MFMA's time, which bounded the kernel; now the
     // splitting's VALU work beside them does as much. Launches, f32 MFMA and this: 6 heads x 1500
     // 53.6 -> 35.9 us, 16 heads x 1037 71.4 -> 43.2, 8 x 12 heads x 1500 600 -> 330 (92 and 167
@@ -659,18 +664,21 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
         }
       }
     };
-    // An element is left to the f32 MFMA when its first part would overflow (from kSplitMax up), or
-    // when the largest of its group of four (of one key, or of one column of V) is below 2^-100:
-    // the MFMA takes parts below 2^-126 as zero, which there would show.
-    constexpr uint32_t kSplitMax = 0x7f7f7fffu, kSplitMin = 0x0d800000u;
-    // the bits of a group's largest magnitude to the running extremes (zero groups count as large)
-    uint32_t ext_hi = 0u, ext_lo = 0xffffffffu;
-    auto extremes = [&](float a, float b, float c, float d) {
-      const uint32_t m = __float_as_uint(fmaxf(fmaxf(fabsf(a), fabsf(b)), fmaxf(fabsf(c), fabsf(d))));
-      ext_hi = max(ext_hi, m);
-      ext_lo = min(ext_lo, m - 1u);
+    constexpr float kSplitMax = 0x1p30f, kSplitMin = 0x1p-40f;
+    // the running extremes of the magnitudes, and of the nonzero ones (as 2 x bits - 1: zero last)
+    float ext_hi = 0.f, ext_lo = kSplitMax;
+    uint32_t ext_nz = 0xffffffffu;
+    auto extremes = [&](f32x4 x) {
+      ext_hi = fmaxf(fmaxf(ext_hi, fabsf(x[0])), fabsf(x[1]));
+      ext_hi = fmaxf(fmaxf(ext_hi, fabsf(x[2])), fabsf(x[3]));
+      ext_lo = fminf(fminf(ext_lo, fabsf(x[0])), fabsf(x[1]));
+      ext_lo = fminf(fminf(ext_lo, fabsf(x[2])), fabsf(x[3]));
     };
-    auto no_parts = [&]() { return ext_hi > kSplitMax || ext_lo < kSplitMin; };
+    auto nonzero = [&](f32x4 x) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ext_nz = min(ext_nz, (__float_as_uint(x[e]) << 1) - 1u);
+    };
+    constexpr uint32_t kNzMin = (uint32_t)(127 - 40) << 24;  // 2 x kSplitMin's bits
     // Split the tile `it` held in kreg / vreg into the LDS planes (V rows past the last valid key
     // zeroed); true if some element has no parts.
     auto store_planes = [&](int it) -> bool {
@@ -683,29 +691,37 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
 #pragma unroll
         for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x2*>(dst + k * PL) = u32x2{lo[k], hi[k]};
       };
-      ext_hi = 0u;
-      ext_lo = 0xffffffffu;
+      ext_hi = 0.f;
+      ext_lo = kSplitMax;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         if constexpr (KT) {
           const int r = 4 * (tid / (BN / 4)) + i, c = tid % (BN / 4);
           put(&kpl[r * BN + 8 * swz_kt(r, c >> 1) + 4 * (c & 1)], kreg[i]);
-          extremes(kreg[0][i], kreg[1][i], kreg[2][i], kreg[3][i]);
         } else {
           const int u = tid + i * NT, r = u / (D / 4), c = u % (D / 4);
           put(&kpl[r * D + 8 * swz_kr(r, c >> 1) + 4 * (c & 1)], kreg[i]);
-          extremes(kreg[i][0], kreg[i][1], kreg[i][2], kreg[i][3]);
         }
+        extremes(kreg[i]);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = 4 * (tid / (D / 4)) + i, c = tid % (D / 4);
+        extremes(vreg[i]);  // (rows past the last valid one hold its values)
         if (!full && kb + r > klast) vreg[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         put(&vpl[r * D + 8 * swz_v(r, c >> 1) + 4 * (c & 1)], vreg[i]);
       }
+      // some element below kSplitMin: whether one that is not zero
+      if (__builtin_amdgcn_ballot_w64(ext_lo < kSplitMin) != 0) {
+        ext_nz = 0xffffffffu;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) extremes(vreg[0][e], vreg[1][e], vreg[2][e], vreg[3][e]);
-      return no_parts();
+        for (int i = 0; i < 4; ++i) {
+          nonzero(kreg[i]);
+          nonzero(vreg[i]);
+        }
+        if (ext_nz < kNzMin) return true;
+      }
+      return ext_hi > kSplitMax;
     };
     // Q: step s, lane group g: d = 16 s + 8 g .. +7 of the lane's row
     u32x4 qs[3][D / 16];
@@ -720,14 +736,16 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
         for (int k = 0; k < 2; ++k) {
           f32x4 x = ld4f<kF32>(qr + 16 * s + 8 * g + 4 * k);
           if (row >= p.Tq) x = f32x4{0.f, 0.f, 0.f, 0.f};
-          extremes(x[0], x[1], x[2], x[3]);
+          extremes(x);
+          nonzero(x);
           split2(x[0], x[1], w[2 * k]);
           split2(x[2], x[3], w[2 * k + 1]);
         }
 #pragma unroll
         for (int k = 0; k < 3; ++k) qs[k][s] = u32x4{w[0][k], w[1][k], w[2][k], w[3][k]};
       }
-      q_big = __builtin_amdgcn_ballot_w64(no_parts()) != 0;
+      // (a scale so large that products below f32's range would show is left to the f32 MFMA too)
+      q_big = __builtin_amdgcn_ballot_w64(ext_hi > kSplitMax || ext_nz < kNzMin) != 0 || sl2 > kSplitMax;
     }
     // transposing reads, as in the 16-bit kernels below
     const int jt = lane & 15;
@@ -754,13 +772,13 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
     };
     if (tid == 0) f32_only = 0;
     __syncthreads();
-    bool redo = false;
+    bool redo = false;  // the same for every wave
     for (int it = t_begin; it < t_end; ++it) {
       const int kb = it * BN;
       // (every wave has finished with the previous tile's planes: the barrier at the loop's end)
       if (store_planes(it) || q_big) f32_only = 1;
       __syncthreads();
-      redo = __builtin_amdgcn_readfirstlane(f32_only) != 0;  // the same for every wave
+      redo = __builtin_amdgcn_readfirstlane(f32_only) != 0;
       if (redo) break;
       f32x16 sacc[QW][2];
 #pragma unroll

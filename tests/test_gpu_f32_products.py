@@ -1,7 +1,7 @@
 """The four-wave f32 kernel's products, each f32 operand the sum of three bf16 parts: errors at the
 level of f32 sums over magnitudes from 2^-112 to 2^112, tile and row remainders in both K layouts,
-operands without such parts (infinite, within half a bf16 step of overflow, or tiny), and masked
-keys of any value."""
+operands without such parts (infinite, huge, or tiny, alone or beside ordinary ones), and
+masked keys of any value."""
 
 from __future__ import annotations
 
@@ -97,6 +97,53 @@ def test_a_tiny_column_beside_others(gpu):
     got = _run(gpu, q, k, v, False, 0.125)
     err = np.linalg.norm(got - want, axis=2) / np.linalg.norm(want, axis=2)
     assert err.max() < 1.2e-6
+
+
+@pytest.mark.parametrize("tiny", [2.0 ** -92, 1.0e-36, 1.2345e-39])
+@pytest.mark.parametrize("k_transposed", [True, False])
+def test_a_tiny_value_beside_others(gpu, tiny, k_transposed):
+    """One tiny value (the last a subnormal) among keys and columns at 1: a causal row that sees its
+    key alone returns it (weight 1, so to the rounding of 1 / l), and every row keeps its error."""
+    rng = np.random.default_rng(650)
+    q, k, v = (randn(rng, (1, 2, n, 64)) for n in (70, 150, 150))
+    v[0, 1, 0, 20] = np.float32(tiny)
+    v[0, 1, 1, 20] = 1.0
+    got = _run(gpu, q, k, v, k_transposed, 0.125, causal=True)
+    want0 = v[:, :, 0].astype(np.float64)
+    assert np.max(np.abs(got[:, :, 0] - want0) / np.abs(want0)) < 3e-7
+    for row in (1, 2, 69):
+        want = _exact(q[:, :, row:row + 1], k[:, :, :row + 1], v[:, :, :row + 1], 0.125)
+        assert np.linalg.norm(got[:, :, row:row + 1] - want) / np.linalg.norm(want) < 1e-6, row
+
+
+@pytest.mark.parametrize("k_transposed", [True, False])
+@pytest.mark.parametrize("tiny,large", [(1.0e-36, 1.0e36), (1.2345e-39, 1.0e38)])
+def test_a_tiny_key_element_against_a_large_query_one(gpu, tiny, large, k_transposed):
+    """Scores that rest on one dimension, tiny in every key and large in every query, the other
+    dimensions ordinary (a subnormal of ~20 bits: its parts are exact, its products f32's)."""
+    rng = np.random.default_rng(660)
+    q, k, v = (randn(rng, (1, 2, n, 64)) for n in (70, 150, 150))
+    q[..., 6] = np.float32(large) * np.sign(q[..., 6])
+    k[..., 6] *= np.float32(tiny)
+    want = _exact(q, k, v, 0.125)
+    got = _run(gpu, q, k, v, k_transposed, 0.125)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 1e-6
+
+
+@pytest.mark.parametrize("k_transposed", [True, False])
+def test_scores_below_the_f32_range_weigh_nothing(gpu, k_transposed):
+    """Finite elements whose products pass -3.4e38, by so much that the products of their parts do
+    too, with either sign: the score is -inf in f32, its weight 0."""
+    rng = np.random.default_rng(680)
+    q, k, v = (randn(rng, (1, 3, n, 64)) for n in (130, 200, 200))
+    q[..., 5] = np.float32(3e21) * (1 + rng.random((1, 3, 130), dtype=np.float32))
+    k[..., 5] = 0.0
+    gone = [3, 64, 100, 199]
+    k[:, :, gone, 5] = np.float32(-3e21) * (1 + rng.random((1, 3, 4), dtype=np.float32))
+    kept = [j for j in range(200) if j not in gone]
+    got = _run(gpu, q, k, v, k_transposed, 0.125)
+    want = _exact(q, k[:, :, kept], v[:, :, kept], 0.125)
+    assert np.linalg.norm(got - want) / np.linalg.norm(want) < 1e-6
 
 
 @pytest.mark.parametrize("k_transposed", [True, False])
