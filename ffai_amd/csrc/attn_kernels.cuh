@@ -563,7 +563,9 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
   };
 
   // f32: mask, online softmax of tile `kb`'s scores (the weights replace them), rescale of O.
-  auto softmax_f32 = [&](f32x16 (&sacc)[QW][2], int kb) {
+  // The reference is a whole number (scales by it are exact). `lift`: a factor for O besides (1, or
+  // once kLift).
+  auto softmax_f32 = [&](f32x16 (&sacc)[QW][2], int kb, float lift) {
     if (kb + BN > kv_end || (p.causal && kb + BN - 1 > p.q_offset + q0)) {
       mask_subtile(sacc, kb, 0);
       mask_subtile(sacc, kb, 1);
@@ -574,13 +576,14 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
 #pragma unroll
       for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(sacc[0][st][r], sacc[0][st][r + 1]));
     const float mx_s = partner_max(mx) * sl2;
-    if (__builtin_amdgcn_ballot_w64(mx_s > m_s[0] + kRescaleSlack) != 0) {
-      const float m_new = fmaxf(m_s[0], mx_s);
+    if (__builtin_amdgcn_ballot_w64(mx_s > m_s[0] + kRescaleSlack || lift != 1.f) != 0) {
+      const float m_new = __builtin_ceilf(fmaxf(m_s[0], mx_s));
       const float corr = fast_exp2(m_s[0] - ((m_new == kNegInf) ? 0.f : m_new));
       m_s[0] = m_new;
       l_run[0] *= corr;
+      const float o_corr = corr * lift;
 #pragma unroll
-      for (int dt = 0; dt < D / 32; ++dt) oacc[0][dt] *= corr;
+      for (int dt = 0; dt < D / 32; ++dt) oacc[0][dt] *= o_corr;
     }
     const float mc = (m_s[0] == kNegInf) ? 0.f : m_s[0];
     float rs = 0.f;
@@ -611,7 +614,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
 #pragma unroll
           for (int e = 0; e < 4; ++e) sacc[0][st] = mfma_f32(a[e], qf[0][4 * j + e], sacc[0][st]);
         }
-      softmax_f32(sacc, kb);
+      softmax_f32(sacc, kb, 1.f);
 #pragma unroll
       for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
@@ -642,6 +645,13 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
     // part products could pass f32's range with either sign), starts over on the f32 MFMA: 8 x 12
     // heads x 1500 547 us if all meet one in their first tile and 842 in their last, 333 in none
     // (578 when the f32 MFMA did all; 6 heads 51, 66, 35 and 50).
+    // A weight below 2^-103 loses at most 2^-118, beside a weight of 1 in its row: with values from
+    // kSplitMin to kSplitMax, 65536 of them do not reach 2^-24 of the row's sum. But a column may
+    // hold zeros where the row's weights are: from the first tile with a zero in V on, the weights
+    // (not l_run) and O are kLift times larger (a power of two: exact), where every normal weight
+    // has its parts (4% more time with a zero in every tile). Raising the exponents by the lift
+    // instead would cost no multiplications, but their rounding: error against 64 bits, 6 heads x
+    // 1500, 5.0e-7 and 3.4e-7.
     // Six bf16 products take 6/16 of the f32 MFMA's time, which bounded the kernel; now the
     // splitting's VALU work beside them does as much. Launches, f32 MFMA and this: 6 heads x 1500
     // 53.6 -> 35.9 us, 16 heads x 1037 71.4 -> 43.2, 8 x 12 heads x 1500 600 -> 330 (92 and 167
@@ -650,7 +660,8 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
     // ---------------------------------------------------------------------------------------
     constexpr int PL = BN * D;  // elements of a plane
     constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
-    __shared__ int f32_only;  // some element has no parts
+    constexpr int kNoParts = 1, kZeroInV = 2;
+    __shared__ int seen;  // of the above, in the tiles so far
     uint16_t* kpl = reinterpret_cast<uint16_t*>(k_lds);
     uint16_t* vpl = reinterpret_cast<uint16_t*>(v_lds);
     // two elements to a packed pair of each part
@@ -665,6 +676,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
       }
     };
     constexpr float kSplitMax = 0x1p30f, kSplitMin = 0x1p-40f;
+    constexpr float kLiftLog2 = 40.f, kLift = 0x1p40f;  // (x 2^8, kRescaleSlack, x kSplitMax x keys: finite)
     // the running extremes of the magnitudes, and of the nonzero ones (as 2 x bits - 1: zero last)
     float ext_hi = 0.f, ext_lo = kSplitMax;
     uint32_t ext_nz = 0xffffffffu;
@@ -680,8 +692,8 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
     };
     constexpr uint32_t kNzMin = (uint32_t)(127 - 40) << 24;  // 2 x kSplitMin's bits
     // Split the tile `it` held in kreg / vreg into the LDS planes (V rows past the last valid key
-    // zeroed); true if some element has no parts.
-    auto store_planes = [&](int it) -> bool {
+    // zeroed); which of kNoParts and kZeroInV this lane's elements show.
+    auto store_planes = [&](int it) -> int {
       const int kb = it * BN, klast = kv_end - 1;
       const bool full = kb + BN <= kv_end;
       auto put = [&](uint16_t* dst, f32x4 x) {
@@ -711,17 +723,19 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
         if (!full && kb + r > klast) vreg[i] = f32x4{0.f, 0.f, 0.f, 0.f};
         put(&vpl[r * D + 8 * swz_v(r, c >> 1) + 4 * (c & 1)], vreg[i]);
       }
-      // some element below kSplitMin: whether one that is not zero
+      // some element below kSplitMin: whether one that is not zero, or a zero in V
       if (__builtin_amdgcn_ballot_w64(ext_lo < kSplitMin) != 0) {
         ext_nz = 0xffffffffu;
+        ext_lo = kSplitMax;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           nonzero(kreg[i]);
           nonzero(vreg[i]);
+          extremes(vreg[i]);
         }
-        if (ext_nz < kNzMin) return true;
+        if (ext_nz < kNzMin) ext_hi = 2.f * kSplitMax;
       }
-      return ext_hi > kSplitMax;
+      return (ext_hi > kSplitMax ? kNoParts : 0) | (ext_lo == 0.f ? kZeroInV : 0);
     };
     // Q: step s, lane group g: d = 16 s + 8 g .. +7 of the lane's row
     u32x4 qs[3][D / 16];
@@ -770,15 +784,18 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
       const u32x2 a0 = lds_tr(base), a1 = lds_tr(base + 8 * D);
       return u32x4{a0.x, a0.y, a1.x, a1.y};
     };
-    if (tid == 0) f32_only = 0;
+    if (tid == 0) seen = 0;
     __syncthreads();
     bool redo = false;  // the same for every wave
+    float w_scale = 1.f;
     for (int it = t_begin; it < t_end; ++it) {
       const int kb = it * BN;
       // (every wave has finished with the previous tile's planes: the barrier at the loop's end)
-      if (store_planes(it) || q_big) f32_only = 1;
+      const int mine = store_planes(it) | (q_big ? kNoParts : 0);
+      if (mine) atomicOr(&seen, mine);
       __syncthreads();
-      redo = __builtin_amdgcn_readfirstlane(f32_only) != 0;
+      const int all = __builtin_amdgcn_readfirstlane(seen);
+      redo = (all & kNoParts) != 0;
       if (redo) break;
       f32x16 sacc[QW][2];
 #pragma unroll
@@ -813,7 +830,13 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
 #pragma unroll
           for (int k = 0; k < 3; ++k) a[t & 1][dt][k] = vfrag(vpl + k * PL, t, dt);
       };
-      softmax_f32(sacc, kb);
+      const float scale_w = (all & kZeroInV) != 0 ? kLift : 1.f;
+      softmax_f32(sacc, kb, scale_w == w_scale ? 1.f : kLift);
+      w_scale = scale_w;
+      if (__builtin_amdgcn_ballot_w64(w_scale != 1.f) != 0) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st) sacc[0][st] *= kLift;
+      }
       // parts of the weights of keys 16 t + 4 g + e (e < 4) and 16 t + 8 + 4 g + e - 4, as they lie
       u32x4 pf[2][3];
       auto split_p = [&](int t) {
@@ -842,6 +865,9 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
       }
       __syncthreads();
     }
+    // (m, l, O) of the lifted O: l lifted too, and the reference as much lower (both exact)
+    l_run[0] *= w_scale;
+    m_s[0] -= w_scale != 1.f ? kLiftLog2 : 0.f;
     if (redo) {
       m_s[0] = kNegInf;
       l_run[0] = 0.f;

@@ -1,7 +1,7 @@
 """The four-wave f32 kernel's products, each f32 operand the sum of three bf16 parts: errors at the
 level of f32 sums over magnitudes from 2^-112 to 2^112, tile and row remainders in both K layouts,
-operands without such parts (infinite, huge, or tiny, alone or beside ordinary ones), and
-masked keys of any value."""
+operands without such parts (infinite, huge, or tiny, alone or beside ordinary ones), weights down
+to the smallest f32 holds, and masked keys of any value."""
 
 from __future__ import annotations
 
@@ -9,10 +9,18 @@ import numpy as np
 import pytest
 import torch
 
+from ffai_amd import _lib as L
 from ffai_amd import flash_attn as fa
 from tests.helpers import randn
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def split_override():
+    prev = L.get_fwd_split_override()
+    yield L.set_fwd_split_override
+    L.set_fwd_split_override(*prev)
 
 
 def _run(gpu, q, k, v, k_transposed, scale, **kw):
@@ -128,6 +136,30 @@ def test_a_tiny_key_element_against_a_large_query_one(gpu, tiny, large, k_transp
     want = _exact(q, k, v, 0.125)
     got = _run(gpu, q, k, v, k_transposed, 0.125)
     assert np.linalg.norm(got - want) / np.linalg.norm(want) < 1e-6
+
+
+@pytest.mark.parametrize("keys,at,pieces", [(64, 9, 1), (200, 9, 1), (200, 150, 1), (200, 150, 4)])
+@pytest.mark.parametrize("log2_weight", [-90, -107, -113, -119, -124])
+def test_small_weights_keep_their_bits(gpu, split_override, log2_weight, keys, at, pieces):
+    """A column whose only nonzero value stands behind a small weight, in the first tile or a later
+    one, the item whole or in pieces: the output is that weight. Its score, ~|log2_weight| in base
+    2, carries 2^-24 of itself from each of the score, scale and exponent roundings, so the weight 3
+    |log2_weight| 2^-24 ln 2 of itself; twice that allowed, and the step of the subnormals."""
+    split_override(-1, pieces)
+    rng = np.random.default_rng(670)
+    q, k, v = (randn(rng, (1, 2, n, 64)) for n in (70, keys, keys))
+    q[...], k[...] = 0.0, 0.0
+    q[..., 0] = 1.0 + rng.random((1, 2, 70), dtype=np.float32) / 64
+    k[..., at, 0] = log2_weight * np.log(2.0)
+    v[..., 33] = 0.0
+    v[..., at, 33] = 1.0
+    want = _exact(q, k, v, 1.0)[..., 33]
+    got = _run(gpu, q, k, v, True, 1.0)[..., 33]
+    kept = want * keys > 2.0 ** -126  # (exp2 flushes a smaller weight)
+    assert kept.any()
+    err = np.max(((np.abs(got - want) - 2.0 ** -149) / want)[kept])
+    print(f"weight 2^{log2_weight}: {err:.2e}")
+    assert err < 6 * abs(log2_weight) * 1.02 * 2.0 ** -24 * np.log(2.0)
 
 
 @pytest.mark.parametrize("k_transposed", [True, False])
