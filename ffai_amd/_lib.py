@@ -113,6 +113,7 @@ def load():
     L.ffai_attn_fwd.argtypes = [dp, vp, vp, vp, vp, vp, sz, vp]
     L.ffai_attn_plan_info.argtypes = [dp, ctypes.POINTER(ctypes.c_int32)]
     L.ffai_attn_row_block.argtypes = [dp]
+    L.ffai_attn_key_groups.argtypes = [dp]
     L.ffai_attn_fwd_noalloc.argtypes = [dp, vp, vp, vp, vp, vp]
     L.ffai_attn_noalloc_plan_info.argtypes = [dp, ctypes.POINTER(ctypes.c_int32),
                                               ctypes.POINTER(sz)]
@@ -162,8 +163,8 @@ def load():
     L.ffai_probe_pipes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, vp, vp]
     for name in ("ffai_probe_empty", "ffai_probe_read", "ffai_probe_pipes", "ffai_attn_serves",
                  "ffai_attn_workspace_bytes", "ffai_attn_fwd",
-                 "ffai_attn_plan_info", "ffai_attn_row_block", "ffai_attn_plan_splits", "ffai_attn_fwd_noalloc",
-                 "ffai_attn_noalloc_plan_info",
+                 "ffai_attn_plan_info", "ffai_attn_row_block", "ffai_attn_key_groups",
+                 "ffai_attn_plan_splits", "ffai_attn_fwd_noalloc", "ffai_attn_noalloc_plan_info",
                  "ffai_serves",
                  "ffai_attend", "ffai_attend_workspace_bytes", "ffai_attend_merged",
                  "ffai_attend_merged_workspace_bytes", "ffai_kv_append", "ffai_kv_gather",
@@ -197,7 +198,8 @@ def plan_info(desc: AttnDesc) -> dict:
            "workgroups": info[4]}
     sp = (ctypes.c_int32 * 3)()
     check(load().ffai_attn_plan_splits(ctypes.byref(desc), sp))
-    out.update(items=sp[0], split_items=(sp[1], sp[2]))
+    out.update(items=sp[0], split_items=(sp[1], sp[2]),
+               key_groups=check(load().ffai_attn_key_groups(ctypes.byref(desc))))
     return out
 
 

@@ -237,6 +237,7 @@ struct Plan {
   int n_items, split_lo, split_hi, sec1_work;
   bool xcd_remap;
   bool x16;       // the four-wave x 64-row shape runs on fwd16_kernel (16x16x32 MFMA)
+  int key_groups;  // fwd: 2 when the four-wave x 32-row shape runs as two key groups (eight waves)
   int xcd_shift;  // log2 of the XCDs the sections are rounded to (0: one)
   int cus;
   size_t ws_bytes;
@@ -525,6 +526,14 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
   }
   const int64_t pieces = (int64_t)(p.split_hi - p.split_lo) * p.n_split;
   p.n_work = (int)(items + pieces - (p.split_hi - p.split_lo));
+  // Two key groups (fwd_kernel) for 16-bit four-wave grids of at most one workgroup per CU, from
+  // five tiles a work on: below that the second group's own start and the merge in LDS cost what
+  // it saves. us with one group / two (head_dim 64, bf16): 20 heads x 1500 rows over 65 keys 6.9 /
+  // 7.5, 192 7.4 / 7.9, 256 8.3 / 8.3, 400 11.6 / 10.8, 800 17.2 / 14.7, 1500 26.7 / 21.7; 12
+  // heads x 1037 in 2 pieces 192 8.9 / 9.4, 400 (4 tiles a piece) 10.8 / 11.0, 800 13.7 / 12.8; 6
+  // heads x 1500 in 3 pieces 400 (3 tiles) 11.0 / 11.4, 800 (5) 12.9 / 12.6, 1500 16.0 / 14.7.
+  p.key_groups = (!f32 && d->head_dim == 64 && p.variant == ffai::kWave4 && p.n_work <= cus &&
+                  p.tiles_per_split >= 5) ? 2 : 1;
   // Dispatch. Causal: rank order (longest first) across all XCDs. Otherwise each section's works
   // go to the XCDs in contiguous runs (one head's query blocks, one item's pieces share an L2);
   // split items at the end of the grid form the second section, so that they are dealt to every
@@ -682,6 +691,7 @@ int run_fwd(const ffai_attn_desc* d, const void* q, const void* k, const void* v
   p.sec1_work = pl.sec1_work;
   p.xcd_shift = pl.xcd_shift;
   p.cus = pl.cus;
+  p.key_groups = pl.key_groups;
   {
     const int xr = 1 << pl.xcd_shift;
     p.sec1_wgs = (pl.sec1_work + xr - 1) / xr * xr;
@@ -867,6 +877,14 @@ int ffai_attn_row_block(const ffai_attn_desc* d) {
   if (rc == FFAI_DECLINED) return 0;
   if (rc != FFAI_OK) return fail(rc, why);
   return row_block_of(d, true);
+}
+
+int ffai_attn_key_groups(const ffai_attn_desc* d) {
+  std::string why;
+  const int rc = check_desc(d, &why);
+  if (rc == FFAI_DECLINED) return 0;
+  if (rc != FFAI_OK) return fail(rc, why);
+  return make_plan(d, true, true).key_groups;
 }
 
 int ffai_attn_noalloc_plan_info(const ffai_attn_desc* d, int32_t info[5], size_t* bytes) {

@@ -43,6 +43,7 @@ struct FwdParams {
   int32_t xcd_remap;
   int32_t xcd_shift;         // log2 of the device's XCD count (sections are whole XCD rounds)
   int32_t cus;               // the device's CUs (host side: launch shaping)
+  int32_t key_groups;        // host side: 2 = the four-wave shape as two key groups of four waves
   int32_t dma;               // 16-bit: whole tiles may go global -> LDS by DMA (K and V aligned,
                              // and each lane's byte offset within one of their tiles fits 32
                              // bits)

@@ -36,9 +36,8 @@ hipError_t pick_variant(const FwdParams& p, int variant, hipStream_t s) {
   switch (variant) {
     case kWave1: return launch_one<MODE, KVT, OUTT, D, KT, 1, 1>(p, s);
     case kWave4:
-      // at most one workgroup per CU: two key groups (see fwd_kernel)
       if constexpr (MODE != kF32 && D == 64)
-        if (p.n_work <= p.cus && p.Tk > kBlockN) return launch_one<MODE, KVT, OUTT, D, KT, 8, 1>(p, s);
+        if (p.key_groups == 2) return launch_one<MODE, KVT, OUTT, D, KT, 8, 1>(p, s);
       return launch_one<MODE, KVT, OUTT, D, KT, 4, 1>(p, s);
     case kWave4x2:
       if constexpr (MODE != kF32 && D == 64) return launch_one<MODE, KVT, OUTT, D, KT, 4, 2>(p, s);

@@ -143,6 +143,12 @@ int ffai_attn_plan_info(const ffai_attn_desc* d, int32_t info[5]);
  * FFAI_ERR_INVALID. */
 int ffai_attn_row_block(const ffai_attn_desc* d);
 
+/* Diagnostic, no counterpart in the reference: the key groups of the fused kernel's workgroups for
+ * `d`: 2 when the shape of four waves x 32 rows (info[1] 1 above) runs as eight waves, the second
+ * four on the second half of a work's keys; else 1. 0 for a decode plan or a declined descriptor,
+ * FFAI_ERR_INVALID for a malformed one. */
+int ffai_attn_key_groups(const ffai_attn_desc* d);
+
 /* Diagnostic, no counterpart in the reference: the plan ffai_attn_fwd_noalloc runs for `d`
  * (info as ffai_attn_plan_info) and the scratch bytes it uses (*bytes, at most
  * ffai_attn_noalloc_scratch_bytes()). Returns as ffai_attn_plan_info. */

@@ -121,6 +121,7 @@ extern "C" {
     pub fn ffai_attn_noalloc_scratch_bytes() -> usize;
     pub fn ffai_attn_plan_info(d: *const ffai_attn_desc, info: *mut i32) -> c_int;
     pub fn ffai_attn_row_block(d: *const ffai_attn_desc) -> c_int;
+    pub fn ffai_attn_key_groups(d: *const ffai_attn_desc) -> c_int;
     pub fn ffai_attn_plan_splits(d: *const ffai_attn_desc, info: *mut i32) -> c_int;
     pub fn ffai_attn_noalloc_plan_info(d: *const ffai_attn_desc, info: *mut i32,
                                        bytes: *mut usize) -> c_int;

@@ -114,3 +114,23 @@ def test_every_work_runs_once_for_every_xcd_count(lib, xcds, args):
     causal = len(args) > 10 and args[10]
     works = _work_map(p["workgroups"], sec1, xcds.bit_length() - 1, not causal)
     assert sorted(works) == list(range(p["workgroups"]))
+
+
+@pytest.mark.parametrize("args,groups", [
+    # a whisper-large-v3 window: 240 works of 24 tiles on 256 CUs
+    ((L.BF16, L.BF16, L.BF16, 1, 20, 20, 1500, 1500, 64, L.K_ROWS), 2),
+    ((L.F16, L.F16, L.F32, 1, 20, 20, 1500, 320, 64, L.K_TRANSPOSED), 2),  # 5 tiles
+    ((L.F16, L.F16, L.F32, 1, 20, 20, 1500, 256, 64, L.K_TRANSPOSED), 1),  # 4
+    ((L.BF16, L.BF16, L.BF16, 1, 20, 20, 1500, 65, 64, L.K_ROWS), 1),
+    ((L.BF16, L.BF16, L.BF16, 1, 6, 6, 1500, 400, 64, L.K_ROWS), 1),   # pieces of 3 tiles
+    ((L.BF16, L.BF16, L.BF16, 1, 6, 6, 1500, 800, 64, L.K_ROWS), 2),   # pieces of 5
+    ((L.BF16, L.BF16, L.BF16, 2, 20, 20, 1500, 1500, 64, L.K_ROWS), 1),  # more works than CUs
+    ((L.BF16, L.BF16, L.BF16, 1, 10, 10, 2900, 1500, 128, L.K_ROWS), 1),  # head_dim 128
+    (TINY32, 1),
+    (CROSS5, 0),  # decode
+])
+def test_key_groups(lib, args, groups):
+    """Two key groups from five tiles a work on, in 16-bit head_dim-64 grids of at most one
+    workgroup per CU."""
+    L.set_geometry_override(256, 8)
+    assert L.plan_info(_desc(lib, *args))["key_groups"] == groups
