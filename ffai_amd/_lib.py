@@ -189,7 +189,11 @@ def gemv_plan_info(out_dim: int, in_dim: int, rows: int) -> dict:
 
 
 def plan_info(desc: AttnDesc) -> dict:
-    """The launch plan ffai_attn_fwd uses for `desc` with vector-aligned operands."""
+    """The launch plan ffai_attn_fwd uses for `desc` with 16-byte-aligned K and V: kernel ("fwd" or
+    "decode"), shape (of the fused kernel, or the decode kernel's waves per workgroup), key splits,
+    tiles per split, workgroups, the fused kernel's items, those that are split and its key groups.
+    "row_block": 0, or the rows of the row blocks that the call runs as on the decode kernel, in
+    place of that plan (which a forced split or launch shape still takes)."""
     info = (ctypes.c_int32 * 5)()
     check(load().ffai_attn_plan_info(ctypes.byref(desc), info))
     kernel = "decode" if info[0] == 1 else "fwd"
@@ -199,13 +203,14 @@ def plan_info(desc: AttnDesc) -> dict:
     sp = (ctypes.c_int32 * 3)()
     check(load().ffai_attn_plan_splits(ctypes.byref(desc), sp))
     out.update(items=sp[0], split_items=(sp[1], sp[2]),
-               key_groups=check(load().ffai_attn_key_groups(ctypes.byref(desc))))
+               key_groups=check(load().ffai_attn_key_groups(ctypes.byref(desc))),
+               row_block=check(load().ffai_attn_row_block(ctypes.byref(desc))))
     return out
 
 
 def noalloc_plan_info(desc: AttnDesc) -> dict:
-    """The launch plan ffai_attn_fwd_noalloc uses for `desc` (vector-aligned operands) and the
-    scratch bytes it takes."""
+    """The launch plan ffai_attn_fwd_noalloc uses for `desc` (16-byte-aligned K and V, no row blocks)
+    and the scratch bytes it takes."""
     info = (ctypes.c_int32 * 5)()
     nbytes = ctypes.c_size_t(0)
     check(load().ffai_attn_noalloc_plan_info(ctypes.byref(desc), info, ctypes.byref(nbytes)))

@@ -343,12 +343,14 @@ bool plan_decode(const ffai_attn_desc* d, bool allow_split, size_t max_ws, const
 // call, fwd_kernel / 16 / 32 rows (head_dim 64 unless said): 16 heads x 227 rows x 1500 keys
 // 15.0 / 8.8 / 11.3; x 300 rows (304 blocks of 16: a second round) 16.7 / 15.0 / 11.4; the same
 // causal over 448 keys 10.7 / 7.8 / 6.4; 12 heads x 600 x 600 12.8 / 11.6 / 8.9; 20 heads x 600 x
-// 600 (380 blocks of 32) 14.3 / 16.3 / 14.9.
+// 600 (380 blocks of 32) 14.3 / 16.3 / 14.9; few keys too (16 heads x 40 rows x 64 keys 4.7 / 3.8).
 // A workgroup's time grows with its keys, which fwd_kernel spreads over the chip: up to 4096 keys
-// at head_dim 64 (8 waves; 6 heads x 40 rows 38.8 / 14.9 / 19.5; at 8192 keys and 16 heads x 64
-// rows 25.0 / 30.3 / 36.5); at head_dim 128 (4 waves) up to 3072 in 16-row blocks (16 heads x 64
-// rows 33.0 / 28.8 / 37.2, at 4096 34.9 / 43.0 / 55.2) and 1536 in 32-row ones (16 heads x 227
-// rows 27.9 / 17.1 / 20.9; 1 head x 2048 causal 26.4 / 22.2 / 28.3).
+// at head_dim 64 (8 waves; 6 heads x 40 rows 38.8 / 14.9 / 19.5; 16 heads x 512 rows, fwd_kernel /
+// 32 rows, at 1500, 3072 and 4096 keys 14.6 / 10.6, 19.5 / 15.1 and 22.7 / 18.6; at 8192 keys and
+// 16 heads x 64 rows 25.0 / 30.3 / 36.5); at head_dim 128 (4 waves) up to 3072 in 16-row blocks (16
+// heads x 64 rows 33.0 / 28.8 / 37.2, at 4096 34.9 / 43.0 / 55.2) and 1536 in 32-row ones (16 heads
+// x 300 rows, fwd_kernel / 32 rows, at 1500 22.8 / 18.9; 16 heads x 227 rows 27.9 / 17.1 / 20.9; 1
+// head x 2048 causal 26.4 / 22.2 / 28.3).
 // A forced launch shape or split (the tuning knobs) keeps the call on its plan.
 int row_block_of(const ffai_attn_desc* d, bool dma_ok) {
   const int group = d->heads_q / d->heads_kv;
@@ -434,10 +436,12 @@ Plan make_plan(const ffai_attn_desc* d, bool allow_split, bool dma_ok,
   // four-wave grids (two workgroups per CU) of fewer items than CUs fill the 512 slots: 6 heads x
   // 1500 36.5 us in 6 pieces against 40.0 in 5, 44.8 in 4 (288 works: a second round), 41.1 in 3,
   // 53.7 in 2 and 91 whole; 16 heads x 1037 44.0 in 3, 55.1 in 4, 56.5 in 2; up to 1024 items they
-  // aim at ~4096 waves (300 items, when the f32 MFMA bounded them: 183 us in 4 pieces against 236
-  // whole, 197 in 2, 211 in 8). One-wave 16-bit grids (prompt steps
-  // past row_block_of's limits, head_dim-128 decode off the DMA's alignment) fill at most the 768 slots of three workgroups per CU (48 KB of LDS
-  // each): the cross-attention of 228 tokens, 128 items, 14.6 us in 6 pieces against 15.4 in 5,
+  // aim at ~4096 waves (288 items of 18 tiles 77.7 in 4 pieces, 73.9 in 3, 83.1 in 2, 87.5 whole; 280
+  // of 27 tiles 108.5, 108.7, 124.4, 134.9; past ~400 items the bound is generous: 480 of 24 tiles
+  // 149.2 in 3, 139.5 whole, 960 of 10 tiles 134.1 in 2, 119.0 whole). One-wave 16-bit grids (prompt
+  // steps past row_block_of's limits, head_dim-128 decode off the DMA's alignment) fill at most the
+  // 768 slots of three workgroups per CU (48 KB of LDS each): the cross-attention of 228 tokens, 128
+  // items, 14.6 us in 6 pieces against 15.4 in 5,
   // 15.7 in 4 and 19.2 in 7 (896 workgroups: a second round). One-wave f32 grids (two per CU)
   // keep about 512 workgroups: f32 decode over 1500 keys, 6 heads: 25.9 us in 24 pieces, 32.7
   // in 8, 193 whole; 80 items: 55.8 in 7, 73.9 in 4, 86.8 in 24.

@@ -184,7 +184,9 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, k_transposed
         return None
     if nbytes.value and (workspace is None or workspace.numel() * workspace.element_size()
                          < nbytes.value):
-        workspace = _workspace(nbytes.value, q.device)
+        # row blocks use none (at head_dim 128 whether the call runs so depends on its alignment)
+        if desc.head_dim != 64 or lib.ffai_attn_row_block(ctypes.byref(desc)) == 0:
+            workspace = _workspace(nbytes.value, q.device)
     rc = lib.ffai_attn_fwd(ctypes.byref(desc), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                            out.data_ptr(),
                            None if workspace is None else workspace.data_ptr(),
@@ -205,9 +207,9 @@ def workspace_bytes(q, k, v, out, **kw) -> int:
 
 
 def plan(q, k, v, out, **kw) -> dict:
-    """The launch plan ffai_attn_fwd uses for these operands (ffai_attn_plan_info), assuming
-    the kernels' vector alignment: kernel, workgroup shape, key splits, tiles per split and
-    workgroups."""
+    """The launch plan ffai_attn_fwd uses for these operands, or the row blocks ("row_block") that
+    it runs as instead: see _lib.plan_info. K and V 16-byte aligned is assumed (at head_dim 64 it does
+    not matter)."""
     desc = make_desc(q, k, v, out, k_transposed=kw.get("k_transposed", False),
                      scale=kw.get("scale", 1.0), causal=kw.get("causal", False),
                      q_offset=kw.get("q_offset", 0), kv_lens=kw.get("kv_lens"))

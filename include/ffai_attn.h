@@ -94,8 +94,10 @@ void ffai_attn_desc_init(ffai_attn_desc* d, int32_t q_dtype, int32_t kv_dtype,
  * (the failure flash_attn.rs:113-125 documents). */
 int ffai_attn_serves(const ffai_attn_desc* d);
 
-/* Device workspace ffai_attn_fwd needs for this descriptor (split counters and split-key
- * partials; zeroed once before first use, see above); 0 if none. */
+/* Device workspace ffai_attn_fwd needs for this descriptor, whatever the operands' alignment
+ * (split counters and split-key partials; zeroed once before first use, see above); 0 if none.
+ * Not below what the plan of ffai_attn_plan_info takes, so a workspace of this size also serves a
+ * call that runs as row blocks (ffai_attn_row_block), which uses none of it. */
 int ffai_attn_workspace_bytes(const ffai_attn_desc* d, size_t* bytes);
 
 /* O = softmax(scale * Q K^T [+ causal mask]) V. Returns FFAI_DECLINED for descriptors
@@ -125,11 +127,12 @@ int ffai_attn_fwd_noalloc(const ffai_attn_desc* d, const void* q, const void* k,
 size_t ffai_attn_noalloc_scratch_bytes(void);
 
 /* Diagnostic, no counterpart in the reference: the launch plan ffai_attn_fwd uses for `d` when
- * K and V are 16-byte aligned (bases and strides; at head_dim 64 whatever they are), so a
- * test or benchmark can state which kernel shape it ran. info[0]: kernel (0 the fused
- * encoder/prefill kernel, 1 the decode kernel); info[1]: workgroup shape (fused: 0 one wave x
- * 32 query rows, 1 four waves x 32 rows, 2 four waves x 64 rows, 3 the same on 16x16x32 MFMA;
- * decode: waves per workgroup);
+ * K and V are 16-byte aligned (bases and strides; at head_dim 64 whatever they are) and
+ * ffai_attn_row_block is 0, so a test or benchmark can state which kernel shape it ran. info[0]:
+ * kernel (0 the fused encoder/prefill kernel, 1 the decode kernel); info[1]: workgroup shape
+ * (fused: 0 one wave x 32 query rows, 1 four waves x 32 rows - eight waves where
+ * ffai_attn_key_groups is 2 -, 2 four waves x 64 rows, 3 the same on 16x16x32 MFMA; decode: waves
+ * per workgroup);
  * info[2]: key splits per work item (1 = no partials); info[3]: 64-key tiles per split;
  * info[4]: workgroups. Where ffai_attn_row_block is not 0 the call runs as row blocks instead, and
  * this is the plan a forced split or launch shape would start from. Returns FFAI_OK, FFAI_DECLINED
@@ -149,16 +152,17 @@ int ffai_attn_row_block(const ffai_attn_desc* d);
  * FFAI_ERR_INVALID for a malformed one. */
 int ffai_attn_key_groups(const ffai_attn_desc* d);
 
-/* Diagnostic, no counterpart in the reference: the plan ffai_attn_fwd_noalloc runs for `d`
- * (info as ffai_attn_plan_info) and the scratch bytes it uses (*bytes, at most
- * ffai_attn_noalloc_scratch_bytes()). Returns as ffai_attn_plan_info. */
+/* Diagnostic, no counterpart in the reference: the plan ffai_attn_fwd_noalloc runs for `d` where
+ * ffai_attn_row_block is 0 (info as ffai_attn_plan_info) and the scratch bytes that plan uses
+ * (*bytes, at most ffai_attn_noalloc_scratch_bytes(); row blocks use none). Returns as
+ * ffai_attn_plan_info. */
 int ffai_attn_noalloc_plan_info(const ffai_attn_desc* d, int32_t info[5], size_t* bytes);
 
 /* Diagnostic, no counterpart in the reference: which work items of the fused kernel's plan for
  * `d` run as key-split pieces. Items are the (batch, head, query block) triples in dispatch rank
  * (head-major; for a causal launch longest first); info[0]: items, info[1], info[2]: the split
  * ranks [info[1], info[2]) (empty when nothing is split), each in info[2] of plan_info's pieces.
- * Zeros for a decode plan. Returns as ffai_attn_plan_info. */
+ * Zeros for a decode plan; row blocks have no such items. Returns as ffai_attn_plan_info. */
 int ffai_attn_plan_splits(const ffai_attn_desc* d, int32_t info[3]);
 
 /* ------------------------------------------------------------------------------------------

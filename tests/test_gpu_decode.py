@@ -356,6 +356,23 @@ def test_row_blocks(gpu, case, dtype, rnd):
         assert err < TOL_BF16
 
 
+def test_eager_row_blocks_take_no_workspace(gpu, monkeypatch):
+    """A prompt-sized call without a workspace runs as row blocks: nothing is allocated or zeroed
+    beside its output, and the plan names the route. A call that splits its keys still gets one."""
+    rng = np.random.default_rng(227)
+    q, k, v = (round_bf16(randn(rng, (1, 16, n, 64))) for n in (227, 1500, 1500))
+    qd, kd, vd = (_dev(x, torch.bfloat16, gpu) for x in (q, k, v))
+    sizes, real = [], fa._workspace
+    monkeypatch.setattr(fa, "_workspace", lambda n, device: sizes.append(n) or real(n, device))
+    out = fa.attention(qd, kd, vd, scale=0.125, out_dtype=torch.float32)
+    assert sizes == [] and fa.plan(qd, kd, vd, out, scale=0.125)["row_block"] == 16
+    want = oracle.attend_general(q, k, v, k_transposed=False, scale=0.125)
+    assert max_abs(_host(out), want) < TOL_BF16
+    few = fa.attention(qd[:, :, :5], kd, vd, scale=0.125, out_dtype=torch.float32)
+    assert len(sizes) == 1 and sizes[0] > 4096
+    assert max_abs(_host(few), want[:, :, :5]) < TOL_BF16
+
+
 @pytest.mark.parametrize("dtype,rnd", [(torch.bfloat16, round_bf16), (torch.float16, round_f16)])
 @pytest.mark.parametrize("h,tq,tk,d,kt", [
     (6, 5, 4, 64, True), (6, 5, 37, 64, True), (12, 3, 1037, 64, True), (3, 20, 449, 64, False),
