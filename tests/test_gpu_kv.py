@@ -184,6 +184,30 @@ def test_cross_cache_build(gpu, k_transposed, out):
     np.testing.assert_array_equal(v.float().cpu().numpy(), want_v)
 
 
+@pytest.mark.parametrize("k_transposed", [True, False])
+@pytest.mark.parametrize("out", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("t,heads,d", [
+    (1, 3, 64), (7, 3, 128), (8, 2, 8), (63, 3, 64), (65, 3, 128), (69, 5, 64), (733, 2, 128),
+    (1037, 3, 64), (1499, 2, 64), (66, 2, 24),
+    (3001, 89, 64),   # 8346 row blocks of V and 4183 64-frame blocks of K^T: past 4096 workgroups
+])
+def test_cross_cache_build_ends_and_alignments(gpu, t, heads, d, out, k_transposed):
+    """K^T rows at every alignment an odd frame count gives them, last blocks of 1 to 63 frames, few
+    frames, head widths off a power of two, more blocks than workgroups: exact, and nothing written
+    past either output."""
+    rng = np.random.default_rng(t * 100 + d)
+    kp, vp = randn(rng, (t, heads * d)), randn(rng, (t, heads * d))
+    shapes = ((heads, d, t) if k_transposed else (heads, t, d), (heads, t, d))
+    bufs = [torch.full((heads * t * d + 64,), 7.0, dtype=TDT[out], device=gpu) for _ in shapes]
+    k, v = (b[:heads * t * d].view(s) for b, s in zip(bufs, shapes))
+    cross_kv_build(_dev(kp, torch.float32, gpu), _dev(vp, torch.float32, gpu), heads, TDT[out],
+                   k_transposed=k_transposed, out=(k, v))
+    want_k, want_v = okv.cross_cache_build(kp, vp, heads, out, k_transposed=k_transposed)
+    np.testing.assert_array_equal(k.float().cpu().numpy(), want_k)
+    np.testing.assert_array_equal(v.float().cpu().numpy(), want_v)
+    assert all(bool(torch.all(b[heads * t * d:] == 7.0)) for b in bufs)
+
+
 def test_beam_decode_over_device_state(gpu):
     """Three beam steps of one decoder layer: each step appends every beam's new K/V, attends
     (self-attention over the beams' caches, cross-attention over a cache built once), then

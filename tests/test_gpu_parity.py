@@ -13,6 +13,7 @@ import torch
 
 import oracle
 from oracle import textbook
+from ffai_amd import _lib as L
 from ffai_amd import flash_attn as fa
 from tests.helpers import TOL_BF16, TOL_F32, max_abs, randn, round_bf16, round_f16
 
@@ -25,6 +26,30 @@ def _dev(x: np.ndarray, dtype, device) -> torch.Tensor:
 
 def _host(t: torch.Tensor) -> np.ndarray:
     return t.float().cpu().numpy()
+
+
+@pytest.fixture(params=["planned", "wave1", "wave4", "wave4x2"])
+def attention(request, gpu):
+    """fa.attention as planned (short grids run as row blocks on the decode kernel), or on the fused
+    kernel in a forced launch shape; "wave4" runs as two key groups in these grids."""
+    lib = L.load()
+    prev = lib.ffai_get_attn_variant()
+    if request.param != "planned":
+        lib.ffai_set_attn_variant(["wave1", "wave4", "wave4x2"].index(request.param))
+
+    def call(q, k, v, out=None, out_dtype=None, **kw):
+        if out is None:
+            out = torch.empty(q.shape, dtype=out_dtype, device=gpu)
+        plan = fa.plan(q, k, v, out, **kw)
+        if request.param != "planned":
+            assert plan["shape"] == request.param and plan["row_block"] == 0, plan
+            if request.param == "wave4":
+                groups = 2 if plan["workgroups"] <= 256 and plan["tiles_per_split"] >= 5 else 1
+                assert plan["key_groups"] == groups, plan
+        return fa.attention(q, k, v, out=out, **kw)
+
+    yield call
+    lib.ffai_set_attn_variant(prev)
 
 
 # ---------------------------------------------------------------------------------------------
@@ -100,7 +125,7 @@ def test_attend_decode_f16_kv(gpu, keys):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("k_transposed", [True, False])
 @pytest.mark.parametrize("out_f32", [True, False])
-def test_encoder_16bit(gpu, dtype, k_transposed, out_f32):
+def test_encoder_16bit(gpu, attention, dtype, k_transposed, out_f32):
     """Encoder shape in bf16/f16 with K x 2 (the whisper-small stress case), ragged T=300."""
     rng = np.random.default_rng(2)
     b, h, t, d = 2, 3, 300, 64
@@ -110,9 +135,9 @@ def test_encoder_16bit(gpu, dtype, k_transposed, out_f32):
     v = rnd(randn(rng, (b, h, t, d)))
     scale = d ** -0.5
     kk = np.ascontiguousarray(np.swapaxes(k, 2, 3)) if k_transposed else k
-    out = fa.attention(_dev(q, dtype, gpu), _dev(kk, dtype, gpu), _dev(v, dtype, gpu),
-                       k_transposed=k_transposed, scale=scale,
-                       out_dtype=torch.float32 if out_f32 else dtype)
+    out = attention(_dev(q, dtype, gpu), _dev(kk, dtype, gpu), _dev(v, dtype, gpu),
+                    k_transposed=k_transposed, scale=scale,
+                    out_dtype=torch.float32 if out_f32 else dtype)
     assert out is not None
     want = oracle.attend_general(q, k, v, k_transposed=False, scale=scale)
     err = max_abs(_host(out), want)
@@ -122,7 +147,7 @@ def test_encoder_16bit(gpu, dtype, k_transposed, out_f32):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("k_transposed", [True, False])
-def test_scores_far_above_the_first_subtile(gpu, dtype, k_transposed):
+def test_scores_far_above_the_first_subtile(gpu, attention, dtype, k_transposed):
     """The 16-bit kernel takes its reference max from each row's first 32 keys and raises it
     only when a subtile's weights would leave [0, 2^64]. Scores here jump twice: by ~58 log2
     units at keys 200-259 (weights near 2^58, accepted as they are) and by ~173 at keys 640-699
@@ -141,8 +166,8 @@ def test_scores_far_above_the_first_subtile(gpu, dtype, k_transposed):
     v = rnd(randn(rng, (b, h, t, d)))
     scale = 0.125
     kk = np.ascontiguousarray(np.swapaxes(k, 2, 3)) if k_transposed else k
-    out = fa.attention(_dev(q, dtype, gpu), _dev(kk, dtype, gpu), _dev(v, dtype, gpu),
-                       k_transposed=k_transposed, scale=scale, out_dtype=torch.float32)
+    out = attention(_dev(q, dtype, gpu), _dev(kk, dtype, gpu), _dev(v, dtype, gpu),
+                    k_transposed=k_transposed, scale=scale, out_dtype=torch.float32)
     got = _host(out)
     assert np.isfinite(got).all()
     want = oracle.attend_general(q, k, v, k_transposed=False, scale=scale)
@@ -153,7 +178,7 @@ def test_scores_far_above_the_first_subtile(gpu, dtype, k_transposed):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("sign", [1.0, -1.0])
-def test_first_subtile_outside_the_fast_window(gpu, dtype, sign):
+def test_first_subtile_outside_the_fast_window(gpu, attention, dtype, sign):
     """A wave takes 0 as its reference max only when every row max of its first 32 keys lies
     in [-64, 32] log2 units. Here every score sits near +-87 log2 units, so the wave keeps the
     first subtile's max instead (well above: weights would overflow; well below: they would
@@ -167,8 +192,8 @@ def test_first_subtile_outside_the_fast_window(gpu, dtype, sign):
     k = rnd(np.float32(sign * 60.0) * u + randn(rng, (b, h, t, d)))
     v = rnd(randn(rng, (b, h, t, d)))
     scale = 0.125
-    out = fa.attention(_dev(q, dtype, gpu), _dev(k, dtype, gpu), _dev(v, dtype, gpu),
-                       scale=scale, out_dtype=torch.float32)
+    out = attention(_dev(q, dtype, gpu), _dev(k, dtype, gpu), _dev(v, dtype, gpu),
+                    scale=scale, out_dtype=torch.float32)
     got = _host(out)
     assert np.isfinite(got).all()
     want = oracle.attend_general(q, k, v, k_transposed=False, scale=scale)
@@ -180,7 +205,7 @@ def test_first_subtile_outside_the_fast_window(gpu, dtype, sign):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("row_max", [-40.0, -20.0])
 @pytest.mark.parametrize("shape", [(2, 64, 300), (1, 2, 300), (1, 16, 200)])
-def test_scores_shifted_far_below_zero(gpu, dtype, row_max, shape):
+def test_scores_shifted_far_below_zero(gpu, attention, dtype, row_max, shape):
     """Softmax ignores a shift shared by every score of a row. Q's dimension 0 is set to c and
     K's dimension 0 to -1 for every key, which moves every score of every row by -c * scale;
     c puts the row maxima near `row_max` log2 units, where exp2 of a raw score is below f16's
@@ -209,8 +234,8 @@ def test_scores_shifted_far_below_zero(gpu, dtype, row_max, shape):
     s_max = (np.einsum("bhtd,bhsd->bhts", qs[:, :, :32], ks[:, :, :32]).max(-1) * scale *
              np.log2(np.e))
     assert np.all(s_max < row_max + 6) and np.all(s_max > row_max - 6), (s_max.min(), s_max.max())
-    out = fa.attention(_dev(qs, dtype, gpu), _dev(ks, dtype, gpu), _dev(v, dtype, gpu),
-                       scale=scale, out_dtype=torch.float32)
+    out = attention(_dev(qs, dtype, gpu), _dev(ks, dtype, gpu), _dev(v, dtype, gpu),
+                    scale=scale, out_dtype=torch.float32)
     got = _host(out)
     assert np.isfinite(got).all()
     want = oracle.attend_general(q, k, v, k_transposed=False, scale=scale)
@@ -220,7 +245,7 @@ def test_scores_shifted_far_below_zero(gpu, dtype, row_max, shape):
 
 
 @pytest.mark.parametrize("k_transposed", [True, False])
-def test_f16_query_beyond_the_folding_range(gpu, k_transposed):
+def test_f16_query_beyond_the_folding_range(gpu, attention, k_transposed):
     """The 16-bit kernel folds scale * log2(e) into Q. With scale 1, f16 query elements above
     65504 / log2(e) ~ 45400 would overflow once folded, so such a wave keeps Q as given and
     scales every score instead."""
@@ -233,9 +258,9 @@ def test_f16_query_beyond_the_folding_range(gpu, k_transposed):
     v = round_f16(randn(rng, (b, h, t, d)))
     assert np.abs(q).max() * 1.4426950408889634 > 65504.0
     kk = np.ascontiguousarray(np.swapaxes(k, 2, 3)) if k_transposed else k
-    out = fa.attention(_dev(q, torch.float16, gpu), _dev(kk, torch.float16, gpu),
-                       _dev(v, torch.float16, gpu), k_transposed=k_transposed, scale=1.0,
-                       out_dtype=torch.float32)
+    out = attention(_dev(q, torch.float16, gpu), _dev(kk, torch.float16, gpu),
+                    _dev(v, torch.float16, gpu), k_transposed=k_transposed, scale=1.0,
+                    out_dtype=torch.float32)
     got = _host(out)
     assert np.isfinite(got).all()
     want = oracle.attend_general(q, k, v, k_transposed=False, scale=1.0)
@@ -265,7 +290,7 @@ def _views_with_high_low_word(gpu, arrays, dtype):
 
 
 @pytest.mark.parametrize("shape", [(2, 3, 300), (8, 16, 512)])
-def test_operands_at_high_addresses(gpu, shape):
+def test_operands_at_high_addresses(gpu, attention, shape):
     """Regression: operands whose addresses have bit 31 of the low word set, through the
     one-wave (B2 H3 T300) and the 4-wave x 2-block (B8 H16 T512) encoder variants."""
     rng = np.random.default_rng(31)
@@ -275,7 +300,7 @@ def test_operands_at_high_addresses(gpu, shape):
     kt = round_bf16(randn(rng, (b, h, d, t)))
     v = round_bf16(randn(rng, (b, h, t, d)))
     buf, (qd, ktd, vd) = _views_with_high_low_word(gpu, [q, kt, v], torch.bfloat16)
-    out = fa.attention(qd, ktd, vd, k_transposed=True, scale=0.125, out_dtype=torch.float32)
+    out = attention(qd, ktd, vd, k_transposed=True, scale=0.125, out_dtype=torch.float32)
     torch.cuda.synchronize()
     del buf
     want = oracle.attend_general(q, kt, v, k_transposed=True, scale=0.125)
@@ -393,7 +418,7 @@ def test_whisper_large_shape_sampled_rows(gpu):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("k_transposed", [True, False])
 @pytest.mark.parametrize("b,h", [(2, 3), (8, 32)])  # one-wave / four-wave x 32, four-wave x 64
-def test_16bit_output_rows_paired_and_unpaired(gpu, dtype, k_transposed, b, h):
+def test_16bit_output_rows_paired_and_unpaired(gpu, attention, dtype, k_transposed, b, h):
     """Head_dim 64 with a 16-bit output: rows that admit 16-byte stores are written by lane
     pairs exchanging halves (whole 8-element runs); rows that do not (here a row stride of 68
     elements: 8-byte but not 16-byte aligned) by each lane's own 4-element runs. Both carry the
@@ -411,11 +436,11 @@ def test_16bit_output_rows_paired_and_unpaired(gpu, dtype, k_transposed, b, h):
     paired = torch.empty(b, h, t, d, dtype=dtype, device=gpu)
     wide = torch.full((b, h, t, 68), 7.0, dtype=dtype, device=gpu)  # 68: 136-byte rows
     unpaired = wide[..., :d]
-    if b == 8:
+    if b == 8 and L.load().ffai_get_attn_variant() < 0:
         assert fa.plan(qd, kd, vd, paired, k_transposed=k_transposed,
                        scale=0.125)["shape"] == "wave4x2"
     for out in (paired, unpaired):
-        fa.attention(qd, kd, vd, k_transposed=k_transposed, scale=0.125, out=out)
+        attention(qd, kd, vd, k_transposed=k_transposed, scale=0.125, out=out)
     assert torch.equal(paired.view(torch.int16), unpaired.contiguous().view(torch.int16))
     assert torch.all(wide[..., d:] == 7.0)  # nothing written past each row's 64 elements
     want = oracle.attend_general(q, k, v, k_transposed=False, scale=0.125)

@@ -31,6 +31,16 @@ def split_override():
     L.set_fwd_split_override(*prev)
 
 
+@pytest.fixture
+def no_row_blocks():
+    """Short grids of prompt or window rows keep their key-split plan on the fused kernel (any forced
+    tiles per decode workgroup does that; eight is what the planner starts from)."""
+    lib = L.load()
+    prev = lib.ffai_get_decode_tiles_per_wg()
+    yield lambda: lib.ffai_set_decode_tiles_per_wg(8)
+    lib.ffai_set_decode_tiles_per_wg(prev)
+
+
 def _dev(x, dtype, device):
     return torch.from_numpy(np.ascontiguousarray(x)).to(device=device, dtype=dtype)
 
@@ -186,21 +196,23 @@ def test_one_workspace_across_split_layouts(gpu, split_override):
         assert _counters_zero(ws)
 
 
-@pytest.mark.parametrize("layout", ["forced", "prompt_cross"])
-def test_pieces_in_graph_replays(gpu, split_override, layout):
+@pytest.mark.parametrize("layout", ["forced", "prompt_cross", "prompt_cross_fused"])
+def test_pieces_in_graph_replays(gpu, split_override, no_row_blocks, layout):
     """A launch with split items captured in a HIP graph: every replay (with eager work and
     synchronisation between replays, new inputs copied in) equals the eager call on the same
     inputs bit for bit, and leaves the counters zero. Past the counters the workspace starts as
     garbage (0xFF): partials are written before they are read. Layouts: 9 of 12 four-wave items
-    forced into 3 pieces (K transposed), and the planner's own layout for a prompt step's
-    cross-attention (228 queries x 16 heads over 1500 keys as rows: one-wave items in 6 pieces,
-    768 workgroups)."""
+    forced into 3 pieces (K transposed), and a prompt step's cross-attention (228 queries x 16
+    heads over 1500 keys as rows) as it runs, in row blocks without pieces, and on the fused
+    kernel in the planner's own layout (one-wave items in 6 pieces, 768 workgroups)."""
     rng = np.random.default_rng(77)
     if layout == "forced":
         b, h, tq, tk, d, kt = 2, 3, 700, 700, 64, True
         split_override(9, 3)
     else:
         b, h, tq, tk, d, kt = 1, 16, 228, 1500, 64, False
+        if layout == "prompt_cross_fused":
+            no_row_blocks()
     q = torch.empty(b, h, tq, d, dtype=torch.bfloat16, device=gpu)
     k = torch.empty((b, h, d, tk) if kt else (b, h, tk, d), dtype=torch.bfloat16, device=gpu)
     v = torch.empty(b, h, tk, d, dtype=torch.bfloat16, device=gpu)
@@ -211,6 +223,7 @@ def test_pieces_in_graph_replays(gpu, split_override, layout):
         assert plan["splits"] == 3 and plan["split_items"][1] - plan["split_items"][0] == 9
     else:
         assert plan["splits"] == 6 and plan["workgroups"] == 768, plan
+        assert plan["row_block"] == (0 if layout == "prompt_cross_fused" else 16)
     nbytes = fa.workspace_bytes(q, k, v, out, **args)
     ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=gpu)
     ws[:COUNTER_BYTES].zero_()
@@ -336,13 +349,18 @@ def _broad_cases(seed, n):
         yield i, b, hq, hkv, tq, tk, d, dtype, causal, ragged, items, pieces, kt, out16
 
 
-def test_broad_seeded_sweep_against_the_oracle(gpu, split_override):
+@pytest.mark.parametrize("row_blocks", [True, False])
+def test_broad_seeded_sweep_against_the_oracle(gpu, split_override, no_row_blocks, row_blocks):
     """400 seeded random calls (see _broad_cases) against the oracle, one process, every fourth
     with misaligned inputs: every output within tolerance and every split counter zero again
-    afterwards."""
+    afterwards. Then those that ran as row blocks once more on the fused kernel."""
     worst, kernels = {}, {}
+    if not row_blocks:
+        no_row_blocks()
     for case in _broad_cases(7, 400):
         i, b, hq, hkv, tq, tk, d, dtype, causal, ragged, items, pieces, kt, out16 = case
+        if not row_blocks and (dtype == "f32" or items or hq // hkv * tq <= 32):
+            continue
         rng = np.random.default_rng(7000 + i)
         tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
         rnd = {"bf16": round_bf16, "f16": round_f16, "f32": lambda x: x}[dtype]
@@ -366,17 +384,21 @@ def test_broad_seeded_sweep_against_the_oracle(gpu, split_override):
         err = max_abs(out.float().cpu().numpy(), want)
         tag = dtype + ("/out16" if out16 else "")
         worst[tag] = max(worst.get(tag, 0.0), err)
-        kernels[plan["kernel"]] = kernels.get(plan["kernel"], 0) + 1
+        kernel = "row blocks" if plan["row_block"] else plan["kernel"]
+        kernels[kernel] = kernels.get(kernel, 0) + 1
         assert err < (TOL_F32 if dtype == "f32" else TOL_BF16), (case, plan, err)
         assert _counters_zero(ws), (case, plan)
     print("kernels", kernels, "worst", {t: f"{e:.2e}" for t, e in worst.items()})
-    assert set(kernels) == {"fwd", "decode"}
+    assert set(kernels) == ({"fwd", "decode", "row blocks"} if row_blocks else {"fwd"})
+    assert kernels["fwd"] >= (150 if row_blocks else 100)
 
 
 @pytest.mark.parametrize("dtype,rnd", [(torch.bfloat16, round_bf16), (torch.float16, round_f16)])
 @pytest.mark.parametrize("h,tq,tk,causal,kt,pieces", [
-    (20, 300, 65, False, False, 1),    # two tiles: one a key group, the second a single key
-    (6, 1500, 320, False, True, 3),    # pieces of two tiles, the last of one: its second group empty
+    (20, 300, 65, False, False, 1),    # two tiles: one key group still
+    (20, 300, 257, False, False, 1),   # five: the second group's last a single key
+    (6, 1500, 320, False, True, 3),    # pieces of two tiles, the last of one: one key group
+    (6, 1500, 704, False, True, 2),    # pieces of six tiles and of five
     (6, 1500, 1500, False, False, 3),  # pieces of 8 tiles
     (12, 1037, 1040, False, True, 1),  # 17 tiles: 9 and 8
     (10, 900, 900, True, False, 1),    # causal: query blocks of 2 to 15 tiles
@@ -396,9 +418,50 @@ def test_two_key_groups(gpu, split_override, h, tq, tk, causal, kt, pieces, dtyp
         out, plan, ws = _run(_dev_at(q, dtype, gpu, 0), _dev_at(kd, dtype, gpu, 0),
                              _dev_at(v, dtype, gpu, 0), out_dtype=dtype, **kw)
         assert plan["shape"] == "wave4" and plan["workgroups"] <= 256
+        assert plan["key_groups"] == (2 if plan["tiles_per_split"] >= 5 else 1)
         want = oracle.attend_general(q, k, v, k_transposed=False, scale=0.125, causal=causal,
                                      kv_lens=None if lens is None else np.array(lens, np.int32))
         err = max_abs(out.float().cpu().numpy(), want)
         print(f"two key groups {h} x {tq} x {tk} lens {lens}: {err:.3e}")
         assert err < TOL_BF16
         assert _counters_zero(ws)
+
+
+_APART = {  # score amplitudes by key, ~1.44 log2 units each, over 0.1 elsewhere
+    "first_58": [(200, 260, 40.0)], "first_173": [(200, 260, 120.0)],
+    "second_58": [(700, 760, 40.0)], "second_173": [(700, 760, 120.0)],
+    "both": [(200, 260, 40.0), (700, 760, 120.0)], "both_down": [(200, 260, 120.0), (700, 760, 40.0)],
+    "all_high": [(0, 1000, 60.0)], "all_low": [(0, 1000, -60.0)],
+    "first_low": [(0, 512, -60.0)], "second_low": [(512, 1000, -60.0)],
+}
+
+
+@pytest.mark.parametrize("dtype,rnd", [(torch.bfloat16, round_bf16), (torch.float16, round_f16)])
+@pytest.mark.parametrize("kt", [True, False])
+@pytest.mark.parametrize("pieces", [1, 2])
+@pytest.mark.parametrize("pattern", _APART)
+def test_two_key_groups_with_scores_apart(gpu, split_override, pattern, pieces, kt, dtype, rnd):
+    """Two key groups that hold different references (jumps of ~58 and ~173 log2 units in one half
+    of the keys, every score near +-87, one half far below the other), merged in LDS, the item whole
+    (halves of 512 and 488 keys) and in two pieces (quarters)."""
+    rng = np.random.default_rng(1000)
+    split_override(-1, pieces)
+    b, h, t, d = 1, 2, 1000, 64
+    u = np.zeros(d, np.float32)
+    u[3] = 1.0
+    amp = np.full(t, 0.1, np.float32)
+    for lo, hi, a in _APART[pattern]:
+        amp[lo:hi] = a
+    q = rnd(8.0 * u + 0.05 * randn(rng, (b, h, t, d)))
+    k = rnd(amp[None, None, :, None] * u + 0.05 * randn(rng, (b, h, t, d)))
+    v = rnd(randn(rng, (b, h, t, d)))
+    kd = np.ascontiguousarray(np.swapaxes(k, 2, 3)) if kt else k
+    out, plan, ws = _run(_dev(q, dtype, gpu), _dev(kd, dtype, gpu), _dev(v, dtype, gpu),
+                         out_dtype=torch.float32, scale=0.125, k_transposed=kt)
+    assert plan["key_groups"] == 2 and plan["row_block"] == 0 and plan["splits"] == pieces
+    got = out.cpu().numpy()
+    assert np.isfinite(got).all()
+    err = max_abs(got, oracle.attend_general(q, k, v, k_transposed=False, scale=0.125))
+    print(f"{pattern} x{pieces} kt{int(kt)} {dtype}: {err:.3e}")
+    assert err < TOL_BF16
+    assert _counters_zero(ws)

@@ -77,7 +77,8 @@ def test_decode_splits_twice(gpu):
 def test_encoder_splits_twice(gpu):
     """whisper-tiny f32 encoder (6 heads x 1500 rows: four-wave blocks with the keys split, ~7
     MB of partials), then a smaller f32 one (2 heads x 300 rows), then a 16-bit prompt-step
-    shape (one-wave blocks, split keys, 228 rows x 16 heads over 1500 frames)."""
+    shape (228 rows x 16 heads over 1500 frames) as row blocks, which use neither workspace nor
+    scratch, and on the fused kernel (one-wave blocks, split keys)."""
     lib = L.load()
     g = torch.Generator(device=gpu).manual_seed(71)
     for heads, t in ((6, 1500), (2, 300)):
@@ -90,10 +91,16 @@ def test_encoder_splits_twice(gpu):
     q = _rand((1, 16, 228, 64), torch.bfloat16, gpu, g)
     kt = _rand((1, 16, 64, 1500), torch.bfloat16, gpu, g)
     v = _rand((1, 16, 1500, 64), torch.bfloat16, gpu, g)
-    o_ws, o_na, nbytes = _both(lib, q, kt, v, k_transposed=True, scale=0.125,
-                               out_dtype=torch.float32)
-    assert nbytes > 0
-    _check(o_ws, o_na, "prompt-step cross-attention")
+    prev = lib.ffai_get_decode_tiles_per_wg()
+    try:
+        for tiles, name in ((prev, "row blocks"), (8, "fused")):  # forced tiles: no row blocks
+            lib.ffai_set_decode_tiles_per_wg(tiles)
+            o_ws, o_na, nbytes = _both(lib, q, kt, v, k_transposed=True, scale=0.125,
+                                       out_dtype=torch.float32)
+            assert nbytes > 0
+            _check(o_ws, o_na, f"prompt-step cross-attention, {name}")
+    finally:
+        lib.ffai_set_decode_tiles_per_wg(prev)
 
 
 @pytest.mark.gpu
