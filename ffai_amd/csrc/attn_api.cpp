@@ -294,17 +294,20 @@ bool plan_decode(const ffai_attn_desc* d, bool allow_split, size_t max_ws, const
   // against 165 unsplit. (Measured on 256 CUs: the bounds scale with the device's CUs.)
   const int64_t kMinWorkgroups = std::max(1, geo.cus / 4), kSplitWorkgroups = std::max(1, geo.cus / 2);
   int64_t tps = max_waves;
-  // A unit that its workgroup's waves cover in one round of tiles stays whole (a split would add
-  // the merge's round trips to one round of loads).
+  // In such a grid a unit of at most eight tiles stays whole: a round of eight waves, or two of the
+  // four at head_dim 128 (a split would add the merge's round trips to a round or two of loads: 1 to
+  // 20 heads x 1 row x 300 to 512 keys at head_dim 128 whole 6.5-7.2 us, in pieces of one tile
+  // 6.6-7.7 and of two 6.8-7.6; x 5 rows 6.5-7.2, 8.8-10.1 and 8.0-8.9).
   // Of a split unit at most eight pieces while a workgroup's waves cover one in a round: the merge
   // reads eight partials per round trip, and few units alone do not fill the chip anyway. 6 heads
   // x 5 beams x 1500 keys in 24 / 12 / 8 / 6 / 4 pieces 12.1 / 7.4 / 6.5 / 6.6 / 7.4 us, 12 heads
   // in 12 / 8 / 6 8.3 / 7.1 / 7.1, f32 queries, 6 heads 9.0 / 7.2 / 6.3 / 6.4 / 7.0; 2 heads x 6
   // rows x 4096 keys at head_dim 128 in 64 / 16 / 8 28.9 / 9.1 / 11.2. 500 keys of 6 to 20 heads
   // x 5 beams: whole 5.6-5.8, in 4 5.9-6.5, in 8 7.1-8.2.
-  if (units * ((n_tiles + tps - 1) / tps) < kMinWorkgroups && n_tiles > max_waves)
-    tps = std::max({n_tiles * units / kSplitWorkgroups,
-                    std::min<int64_t>(max_waves, (n_tiles + 7) / 8), int64_t(2)});
+  if (units * ((n_tiles + tps - 1) / tps) < kMinWorkgroups)
+    tps = n_tiles <= 8 ? n_tiles
+                       : std::max(n_tiles * units / kSplitWorkgroups,
+                                  std::min<int64_t>(max_waves, (n_tiles + 7) / 8));
   // a tuning knob (ffai_set_decode_tiles_per_wg / FFAI_DECODE_TILES_PER_WG) may force it
   const int forced_tps = decode_tiles_per_wg();
   if (forced_tps > 0) tps = forced_tps;

@@ -486,6 +486,8 @@ def test_one_wave_grids_stay_within_one_round(lib):
     (6, 5, 512, 64, 1, 8),      # eight waves cover it in a round
     (6, 5, 513, 64, 5, 2), (12, 5, 900, 64, 8, 2), (4, 6, 2048, 64, 8, 4),
     (2, 6, 256, 128, 1, 4), (2, 6, 1024, 128, 8, 2), (2, 6, 4096, 128, 16, 4),
+    (2, 1, 300, 128, 1, 5), (20, 5, 512, 128, 1, 8), (2, 1, 513, 128, 5, 2),  # two rounds of four
+    (40, 5, 512, 128, 2, 4),    # a longer grid: four waves' tiles a workgroup
     (2, 6, 16384, 64, 32, 8),   # past one round of tiles a workgroup, more pieces again
 ])
 def test_decode_pieces_fit_one_merge_round(lib, heads, rows, keys, head_dim, splits, tiles):
