@@ -47,7 +47,8 @@ namespace {
 //   QW    32-query column blocks per wave.
 //   WAVES 8: two key groups of four waves, the second on the second half of the work's keys
 //         through its own tile ring; the first merges the two in LDS. For grids of at most one
-//         workgroup per CU, which otherwise leave one wave to a SIMD and nothing to cover its
+//         workgroup per CU and five tiles or more a work (the planner's rule, key_groups), which
+//         otherwise leave one wave to a SIMD and nothing to cover its
 //         chain of LDS, product and exp latencies; a second workgroup's worth of key pieces
 //         instead pays their merge through memory. 20 heads x 1500 frames (240 items) bf16: 28.6
 //         us with one group, 26.9 in 2 pieces, 23.6 so; 12 heads 26.5 and 21.3; 20 heads x 800
