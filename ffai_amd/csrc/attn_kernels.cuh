@@ -646,7 +646,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
     // part products could pass f32's range with either sign), starts over on the f32 MFMA: 8 x 12
     // heads x 1500 547 us if all meet one in their first tile and 842 in their last, 333 in none
     // (578 when the f32 MFMA did all; 6 heads 51, 66, 35 and 50).
-    // A weight below 2^-103 loses at most 2^-118, beside a weight of 1 in its row: with values from
+    // A weight below 2^-103 loses at most 2^-118, beside one above 1/2 in its row: with values from
     // kSplitMin to kSplitMax, 65536 of them do not reach 2^-24 of the row's sum. But a column may
     // hold zeros where the row's weights are: from the first tile with a zero in V on, the weights
     // (not l_run) and O are kLift times larger (a power of two: exact), where every normal weight
@@ -677,7 +677,8 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
       }
     };
     constexpr float kSplitMax = 0x1p30f, kSplitMin = 0x1p-40f;
-    constexpr float kLiftLog2 = 40.f, kLift = 0x1p40f;  // (x 2^8, kRescaleSlack, x kSplitMax x keys: finite)
+    // (kLift x 2^8, kRescaleSlack, x kSplitMax x any number of keys is finite)
+    constexpr float kLiftLog2 = 40.f, kLift = 0x1p40f;
     // the running extremes of the magnitudes, and of the nonzero ones (as 2 x bits - 1: zero last)
     float ext_hi = 0.f, ext_lo = kSplitMax;
     uint32_t ext_nz = 0xffffffffu;
@@ -691,7 +692,7 @@ __global__ __launch_bounds__(WAVES * 64, (WAVES >= 4 && (D == 64 || MODE != kF32
 #pragma unroll
       for (int e = 0; e < 4; ++e) ext_nz = min(ext_nz, (__float_as_uint(x[e]) << 1) - 1u);
     };
-    constexpr uint32_t kNzMin = (uint32_t)(127 - 40) << 24;  // 2 x kSplitMin's bits
+    constexpr uint32_t kNzMin = ((uint32_t)(127 - 40) << 24) - 1u;  // kSplitMin's
     // Split the tile `it` held in kreg / vreg into the LDS planes (V rows past the last valid key
     // zeroed); which of kNoParts and kZeroInV this lane's elements show.
     auto store_planes = [&](int it) -> int {

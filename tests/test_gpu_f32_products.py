@@ -58,15 +58,37 @@ def test_remainders(gpu, queries, keys, k_transposed):
 
 @pytest.mark.parametrize("e", [-100, -60, -20, 20, 60, 100])
 def test_magnitudes(gpu, e):
-    """Keys and values 2^e times wider (queries 2^-e), and values spread over 2^+-12 within a row:
-    parts are relative to each element, so no magnitude loses bits (below 2^-100, where the third
-    part would underflow, on the f32 MFMA)."""
+    """Keys and values 2^e times wider (queries 2^-e), and values spread over 2^+-12 within a row: no
+    magnitude loses bits (elements outside 2^-40 .. 2^30 send their workgroup to the f32 MFMA)."""
     rng = np.random.default_rng(600 + e)
     q, k, v = (randn(rng, (1, 2, n, 64)) for n in (96, 200, 200))
     v *= np.exp2(rng.integers(-12, 13, size=v.shape)).astype(np.float32)
     q, k, v = np.ldexp(q, -e), np.ldexp(k, e), np.ldexp(v, e)
     want = _exact(q, k, v, 0.125)
     got = _run(gpu, q, k, v, True, 0.125)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"2^{e}: {err:.2e}")
+    assert err < 1e-6
+
+
+@pytest.mark.parametrize("k_transposed", [True, False])
+@pytest.mark.parametrize("e", [-28, -14, 14, 22])
+def test_magnitudes_in_bf16_parts(gpu, e, k_transposed):
+    """As above with every element from 2^-38 to 2^30, so that the products stay on bf16 parts, at
+    either end of their range; queries and keys up to both ends as well."""
+    rng = np.random.default_rng(630 + e)
+
+    def draw(n, spread):
+        x = randn(rng, (1, 2, n, 64))
+        x = np.copysign(np.clip(np.abs(x), 2.0 ** -6, 8.0), x)
+        return np.ldexp(x, rng.integers(-spread, spread + 1, size=x.shape)).astype(np.float32)
+
+    q, k, v = np.ldexp(draw(96, 0), -e), np.ldexp(draw(200, 0), e), np.ldexp(draw(200, 4), e)
+    for x in (q, k, v):
+        assert np.abs(x).min() >= 2.0 ** -38 and np.abs(x).max() <= 2.0 ** 31
+    v = np.clip(v, -2.0 ** 30, 2.0 ** 30)
+    want = _exact(q, k, v, 0.125)
+    got = _run(gpu, q, k, v, k_transposed, 0.125)
     err = np.linalg.norm(got - want) / np.linalg.norm(want)
     print(f"2^{e}: {err:.2e}")
     assert err < 1e-6
